@@ -202,6 +202,20 @@ int omni_prefill_attention_gqa_halves(const void* q, int q_stride, const void* k
                                       int n_heads, int n_kv_heads, int head_dim, float scale,
                                       void* stream);
 
+/* The omni_prefill_attention attention on 32-row tiles of (token, query head) pairs: a
+ * workgroup takes one query block and one KV head, (rows, groups) = (128, 1), (128, 2),
+ * (64, 4) or (32, 8): so many rows of it (qblocks counts are at most
+ * rows / (n_heads / n_kv_heads) tokens), its keys dealt to so many groups of waves whose
+ * softmax states merge in fp32 (the same cache/kv_prealloc.py:181-203 call).  -2 for
+ * scale <= 0 or more query heads per KV head than rows; q, pool and out 16-byte aligned,
+ * out_stride % 8 == 0. */
+int omni_prefill_attention_rows(const void* q, int q_stride, const void* k_cache,
+                                const void* v_cache, int pool_rows, int max_len,
+                                const int64_t* slots, const int64_t* kv_len, const int* qblocks,
+                                int nqb, void* out, int out_stride, int n_heads, int n_kv_heads,
+                                int head_dim, float scale, int rows, int groups,
+                                void* stream);
+
 /* ---------------------------------------------------------------- linears */
 
 /* Epilogues of the skinny GEMMs. */

@@ -2,30 +2,29 @@
 
 ``prefill_attention_pool`` is the varlen causal attention of the packed prefill
 (omniserve/cache/kv_prealloc.py:181-203) over K/V already written to the pool: the host
-cuts every segment into query blocks of consecutive tokens and picks one of four kernels:
+cuts every segment into query blocks of consecutive tokens and picks a kernel by the number
+of workgroups and the longest context (``prefill_plan``):
 
-* <= 32-token blocks, one workgroup per (block, KV head) sharing every K/V tile among the
-  group's query heads: omni_prefill_attention_gqa_halves (the block's key tiles split
-  between two groups of four waves, merged in LDS; <= 6 query heads per KV head) when the
-  longest segment has >= 256 tokens and the workgroups fill half the GPU, else
-  omni_prefill_attention_gqa (four waves) when they fill all of it (one wave per SIMD
-  leaves its softmax's latency unhidden, so with fewer workgroups the per-head kernels are
-  faster);
-* otherwise <= 16-token blocks, one (block, query head) item each:
-  omni_prefill_attention_split (the item's key tiles split over the four waves of a
-  workgroup, states merged in LDS) for up to 4 items per CU, omni_prefill_attention (one
-  wave per item) beyond that.
+* omni_prefill_attention_rows, nearly everywhere: a workgroup takes one KV head's (token,
+  query head) rows of a block in 32-row tiles, (rows, key groups) = (128, 1), (128, 2),
+  (64, 4) or (32, 8): fewer rows per workgroup and more key groups the fewer rows there are;
+* omni_prefill_attention_split (<= 16-token blocks, one (block, query head) item per
+  workgroup, its key tiles split over four waves) for the shortest contexts, where the rows
+  kernel's longer start and merge show;
+* omni_prefill_attention (one wave per item) and its split form, whose accesses ask for no
+  alignment, for what the rows kernel does not take: more than 32 query heads per KV head,
+  scale <= 0, operands off a 16-byte boundary.
 
-MI355X, 12 heads / 2 KV heads, us per launch (per-wave / split / shared-tile / two-group
-shared-tile): one 256-token prompt 13.1 / 6.4 / 24.3 / 23.7; 1 x 1024 39.7 / 32.7 / 79.7 /
-57.4; 1 x 2048 101.3 / 109.5 / 152.8 / 103.0; 1 x 4096 285.1 / 404.0 / 302.2 / 195.2;
-2 x 2048 160.9 / 197.5 / 154.8 / 105.3; 4 x 1024 99.7 / 93.8 / 81.9 / 59.9; 8 x 512 63.7 /
-48.8 / 45.2 / 37.5; 16 x 512 96.8 / 88.6 / 86.7 / 73.9; 8 x 384 33.6 / 31.1 / 34.8 / 31.2;
-16 x 256 33.5 / 33.8 / 26.7 / 26.2; 64 x 128 38.1 / 54.6 / 35.0 / 40.3; 128 x 64 28.5 /
-46.8 / 25.4 / 34.8; a 256-token chunk appended to 1792 keys 72.0 / 22.6 / 152.3 / 101.9;
-32 single tokens at 2048 keys 75.1 / 42.5 / 148.8 / 99.7.  The per-wave and shared-tile
-kernels give identical outputs; the split ones agree with them to the fp16 rounding of the
-probabilities (and, for the two-group kernel, of the second group's output).
+MI355X, 12 heads / 2 KV heads, us per launch, rows (128, 1) / (128, 2) / (64, 4) / (32, 8),
+then the best of the per-wave, split and shared-tile kernels: one 4096-token prompt 86.8 /
+69.4 / 90.3 / 123.7, 193; 1 x 2048 43.2 / 34.9 / 29.1 / 42.8, 98.5; 1 x 1024 24.1 / 20.5 /
+16.1 / 17.8, 31.7; 1 x 512 14.7 / 13.4 / 10.9 / 9.3, 13.8; 1 x 256 9.8 / 10.0 / 8.5 / 7.5,
+6.5; 2 x 2048 54.8 / 39.7 / 56.5 / 81.8, 105; 4 x 1024 33.5 / 33.5 / 40.4 / 60.0, 59; 8 x 512
+22.6 / 24.4 / 32.8 / 48.7, 37; 16 x 256 16.6 / 20.0 / 28.4 / 43.8, 26; 64 x 64 11.6 / 16.9 /
+24.7 / 40.4, 12.7; 4 x 256 10.2 / 10.3 / 8.8 / 13.3, 12.4; 16 x 24 6.5 / 7.7 / 6.8 / 6.7, 4.5;
+a 256-token chunk at 1792 keys 42.4 / 33.9 / 25.9 / 19.3, 22.5; a 1024-token chunk at 3000
+keys 78.3 / 61.0 / 46.4 / 56.1, 107; 32 single tokens at 2048 keys 40.8 / 33.1 / 27.1 / 21.0,
+42.
 """
 
 from __future__ import annotations
@@ -36,13 +35,11 @@ from ._lib import call, ptr, stream
 from .hostio import to_device
 
 QBLOCK = 16
-QBLOCK_GQA = 32
-# (block, head) items per CU up to which the key-split kernel runs (0: never)
+QBLOCK_GQA = 32          # blocks of the shared-tile kernels
+# the rows kernel's most query heads per KV head
+ROWS_MAX_GROUP = 32
+# (block, head) items per CU up to which the split kernel, not the per-wave one, runs
 SPLIT_ITEMS_PER_CU = 4
-# the two-group shared-tile kernel: query heads per KV head it is built for, and the
-# longest segment from which it runs
-HALVES_MAX_GROUP = 6
-HALVES_MIN_SEG = 256
 
 
 _CUS = {}
@@ -65,31 +62,65 @@ def query_blocks(seg_lengths, device, block: int = QBLOCK) -> torch.Tensor:
     return to_device(blocks, torch.int32, device).reshape(-1, 2)
 
 
+def prefill_plan(seg_lengths, starts, nh: int, nkv: int, cus: int) -> tuple:
+    """(entry point, tokens per query block, extra arguments) for segments of seg_lengths
+    tokens appended at starts, in 16-byte aligned tensors (see the module docstring for what
+    each form measures)."""
+    group = nh // nkv
+    blocks = lambda n: sum(-(-L // n) for L in seg_lengths)
+    wgs = lambda rows: blocks(rows // group) * nkv
+    keys = max(st + L for st, L in zip(starts, seg_lengths))
+    items = blocks(QBLOCK) * nh
+    if group > ROWS_MAX_GROUP:
+        return fallback_plan(seg_lengths, nh, cus)
+    # A few short contexts: the split kernel starts and merges in 2-3 us less (1 x 256: 6.5
+    # against 7.5 us, 16 x 24: 4.5 against 6.5) until its items queue (2 x 256: 9.0 against
+    # 7.6) or the keys are many (a 128-token chunk at 500 keys: level).
+    if (keys <= 320 and items <= cus) or (keys <= 64 and items <= 2 * cus):
+        return ("omni_prefill_attention_split", QBLOCK, ())
+    # Rows to spare for every CU only in 128s: fewer rows per workgroup while those still fit
+    # one round of the CUs, with the keys dealt to as many groups as the waves allow.  A long
+    # context takes 64 rows also where they are more than one round but 128 would leave CUs
+    # idle: the last blocks' chain of key tiles is what counts (1 x 2048: 29.1 against 34.9).
+    if wgs(32) <= cus:
+        form = (32, 8)
+    elif wgs(64) <= cus or (wgs(128) < cus and keys >= 1024):
+        form = (64, 4)
+    elif keys > 1024 and wgs(128) < 4 * cus:
+        form = (128, 2)      # 2 x 2048: 39.7 against 54.8 us in one group
+    else:
+        form = (128, 1)      # short chains, or workgroups enough: 8 x 512 22.6 against 24.4
+    return ("omni_prefill_attention_rows", form[0] // group, form)
+
+
+def fallback_plan(seg_lengths, nh: int, cus: int) -> tuple:
+    """The kernels that take any head grouping, scale sign and operand alignment."""
+    items = sum(-(-L // QBLOCK) for L in seg_lengths) * nh
+    split = items <= SPLIT_ITEMS_PER_CU * cus
+    return ("omni_prefill_attention_split" if split else "omni_prefill_attention", QBLOCK, ())
+
+
 def prefill_attention_pool(writer, q: torch.Tensor, layer_idx: int, scale: float,
                            out: torch.Tensor, q_stride: int | None = None) -> torch.Tensor:
     """Causal attention of the writer's packed tokens over their pool rows."""
     pool = writer.pool
     nh = pool.n_heads
-    plan = getattr(writer, "_attn_plan", None)
+    plans = getattr(writer, "_attn_plan", None)
+    if plans is None:
+        plans = writer._attn_plan = {}
+    qp, op = q.data_ptr(), out.data_ptr()
+    plain = bool((qp | op) & 15) or not scale > 0
+    plan = plans.get(plain)
     if plan is None:
         cus = _num_cus(q.device)
-        nqb32 = sum(-(-L // QBLOCK_GQA) for L in writer.seg)
-        items32 = nqb32 * pool.n_kv_heads
-        group = nh // pool.n_kv_heads
-        if (group <= HALVES_MAX_GROUP and max(writer.seg) >= HALVES_MIN_SEG
-                and 2 * items32 >= cus):
-            plan = ("omni_prefill_attention_gqa_halves",
-                    query_blocks(writer.seg, q.device, QBLOCK_GQA))
-        elif items32 >= cus and group <= 8:
-            plan = ("omni_prefill_attention_gqa", query_blocks(writer.seg, q.device, QBLOCK_GQA))
+        if plain:
+            fn, block, extra = fallback_plan(writer.seg, nh, cus)
         else:
-            qb = query_blocks(writer.seg, q.device, QBLOCK)
-            split = qb.shape[0] * nh <= SPLIT_ITEMS_PER_CU * cus
-            plan = ("omni_prefill_attention_split" if split else "omni_prefill_attention", qb)
-        writer._attn_plan = plan
-    fn, qb = plan
-    call(fn, ptr(q), q_stride or q.stride(0), ptr(pool.k[layer_idx]),
+            fn, block, extra = prefill_plan(writer.seg, writer.starts, nh, pool.n_kv_heads, cus)
+        plan = plans[plain] = (fn, query_blocks(writer.seg, q.device, block), extra)
+    fn, qb, extra = plan
+    call(fn, qp, q_stride or q.stride(0), ptr(pool.k[layer_idx]),
          ptr(pool.v[layer_idx]), pool.max_batch, pool.max_len, ptr(writer.token_slot),
-         ptr(writer.kv_len), ptr(qb), qb.shape[0], ptr(out), nh * pool.head_dim, nh,
-         pool.n_kv_heads, pool.head_dim, float(scale), stream())
+         ptr(writer.kv_len), ptr(qb), qb.shape[0], op, nh * pool.head_dim, nh,
+         pool.n_kv_heads, pool.head_dim, float(scale), *extra, stream())
     return out

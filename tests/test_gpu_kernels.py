@@ -296,6 +296,61 @@ def test_prefill_attention_append(gpu, ctx, chunk):
         assert d <= 4e-3, (fn, d)
 
 
+@pytest.mark.parametrize("nh,nkv", [(12, 2), (28, 4), (3, 3), (32, 1)])
+@pytest.mark.parametrize("form", [(128, 1), (128, 2), (64, 4), (32, 8)])
+def test_prefill_attention_rows(gpu, nh, nkv, form):
+    """The row-tile kernel in every form against the oracle: chunk ends on both sides of its
+    32- and 64-key tiles, contexts shorter than its key groups, single tokens, blocks that
+    fill a 32-row tile and that leave one row of it, several query heads per KV head and one.
+    Pool rows past a context hold NaN: nothing beyond a block's last key may be read.
+    Tolerance: the fp16 rounding of P (2^-11 relative on each probability, V ~ N(0, 1)) and of
+    the output, as for the other prefill kernels."""
+    from omniserver_amd.attention import query_blocks
+    from omniserver_amd._lib import call, ptr, stream
+    rows, groups = form
+    if nh // nkv > rows:
+        pytest.skip("more query heads than rows")
+    hd, ML = 128, 640
+    segs = [(0, 1), (0, 33), (31, 1), (63, 2), (64, 1), (200, 97), (0, 130), (511, 129)]
+    say(f"prefill_attention_rows nh={nh} nkv={nkv} form={form}")
+    P, T = len(segs), sum(L for _, L in segs)
+    q = f16((T, nh * hd), 67)
+    kp, vp = f16((P, ML, nkv, hd), 68), f16((P, ML, nkv, hd), 69)
+    slot = torch.tensor([s for s, (_, L) in enumerate(segs) for _ in range(L)])
+    kvl = torch.tensor([st + i + 1 for st, L in segs for i in range(L)])
+    e = ref.decode_attention(q.float().view(T, nh, hd), kp.float(), vp.float(), slot, kvl, hd ** -0.5)
+    for s, (st, L) in enumerate(segs):
+        kp[s, st + L:] = float("nan")
+        vp[s, st + L:] = float("nan")
+    qb = query_blocks([L for _, L in segs], gpu, rows // (nh // nkv))
+    out = torch.full((T, nh, hd), float("nan"), device=gpu, dtype=torch.float16)
+    qg, kg, vg, sg, lg = (t.to(gpu) for t in (q, kp, vp, slot, kvl))
+    call("omni_prefill_attention_rows", ptr(qg), nh * hd, ptr(kg), ptr(vg), P, ML, ptr(sg), ptr(lg),
+         ptr(qb), qb.shape[0], ptr(out), nh * hd, nh, nkv, hd, hd ** -0.5, rows, groups, stream())
+    torch.cuda.synchronize()
+    d = (out.cpu().float() - e).abs().max().item()
+    assert d <= 4e-3, d
+
+
+def test_prefill_attention_pool_unaligned(gpu):
+    """An output off the 16-byte boundary the row-tile kernel needs still runs, on the kernels
+    that ask for none, and agrees with the aligned call to the rounding of P."""
+    from omniserver_amd.attention import prefill_attention_pool
+    from omniserver_amd.kv_cache import PreallocatedKVCache
+    say("prefill_attention_pool unaligned")
+    pool = PreallocatedKVCache(1, 2, 2, 512, 128, gpu, n_heads=12)
+    pool.storage.copy_(f16(tuple(pool.storage.shape), 70))
+    w = pool.mixed_cache([0, 1], [300, 70], [100, 0])
+    q = f16((370, 12 * 128), 71).to(gpu)
+    outs = []
+    for off in (0, 1):
+        buf = torch.zeros(370 * 12 * 128 + 8, device=gpu, dtype=torch.float16)
+        out = buf[off:off + 370 * 12 * 128].view(370, 12, 128)
+        prefill_attention_pool(w, q, 0, 128 ** -0.5, out)
+        outs.append(out.cpu().float())
+    assert (outs[0] - outs[1]).abs().max().item() <= 4e-3
+
+
 # ----------------------------------------------------------------------------- linears
 def _gptq(K, N, seed):
     from omniserver_amd.synth import gptq_random

@@ -412,3 +412,29 @@ def test_prefill_k_slices():
             slices = lib().omni_gemm_slices(K, s)
             assert tiles * slices <= 256 or s == 1, (M, N, K, s)
             assert K // 128 // slices >= 2, (M, N, K, s)
+
+
+def test_prefill_plan_covers_every_call():
+    """Every segment layout gets a kernel whose limits it meets: blocks of at least one token
+    whose rows fit the workgroup, and the unaligned / many-head fallback where the row-tile
+    kernel does not apply."""
+    import random
+    from omniserver_amd.attention import QBLOCK, fallback_plan, prefill_plan
+    rng = random.Random(5)
+    forms = set()
+    for _ in range(400):
+        nkv = rng.choice([1, 2, 4, 8])
+        group = rng.choice([1, 2, 6, 7, 16, 32, 33, 40])
+        segs = [int(2 ** rng.uniform(0, 12)) for _ in range(rng.choice([1, 1, 2, 5, 16, 64]))]
+        starts = [rng.choice([0, 0, 700, 3000]) for _ in segs]
+        fn, block, extra = prefill_plan(segs, starts, nkv * group, nkv, 256)
+        if fn == "omni_prefill_attention_rows":
+            assert extra in ((128, 1), (128, 2), (64, 4), (32, 8))
+            assert group <= 32 and block >= 1 and block * group <= extra[0]
+            forms.add(extra)
+        else:
+            assert fn in ("omni_prefill_attention", "omni_prefill_attention_split")
+            assert block == QBLOCK and extra == ()
+            if group > 32:
+                assert (fn, block, extra) == fallback_plan(segs, nkv * group, 256)
+    assert len(forms) == 4
