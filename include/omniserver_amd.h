@@ -412,6 +412,11 @@ int omni_vit_attention(const void* qkv, int ld, int S, int n_heads, int head_dim
                        const int* cu_seqlens, const int* tiles, int ntiles, void* out, int ldo,
                        float scale, void* stream);
 
+/* omni_vit_attention with tiles in steps of rows = 64 or 128 queries. */
+int omni_vit_attention_rows(const void* qkv, int ld, int S, int n_heads, int head_dim,
+                            const int* cu_seqlens, const int* tiles, int ntiles, void* out,
+                            int ldo, float scale, int rows, void* stream);
+
 /* ---------------------------------------------------------------- fp8 (W8A8) */
 
 /* Row-wise e4m3fn quantisation: scale[r] = amax_k |x[r, k]| / 448 (max(., clamp_min) when

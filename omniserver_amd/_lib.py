@@ -79,6 +79,7 @@ SIGNATURES = {
     "omni_f16_gemm_pipe_packed": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P],
     "omni_vision_rope": [_P, _I, _I, _I, _I, _P, _P, _P],
     "omni_vit_attention": [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _F, _P],
+    "omni_vit_attention_rows": [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _F, _I, _P],
     "omni_gemm_slices": [_I, _I],
     "omni_lmhead_argmax_grid": [_I],
     "omni_lmhead_max_rows": [_I],

@@ -45,7 +45,7 @@ SPLIT_ITEMS_PER_CU = 4
 _CUS = {}
 
 
-def _num_cus(device) -> int:
+def num_cus(device) -> int:
     if device not in _CUS:
         _CUS[device] = torch.cuda.get_device_properties(device).multi_processor_count
     return _CUS[device]
@@ -112,7 +112,7 @@ def prefill_attention_pool(writer, q: torch.Tensor, layer_idx: int, scale: float
     plain = bool((qp | op) & 15) or not scale > 0
     plan = plans.get(plain)
     if plan is None:
-        cus = _num_cus(q.device)
+        cus = num_cus(q.device)
         if plain:
             fn, block, extra = fallback_plan(writer.seg, nh, cus)
         else:

@@ -8,7 +8,7 @@
 // the merger's ln_q at :128), the fused rotary of kernels/vision_rope.py:19-47, and
 // the varlen flash call at :58-63 (cu_seqlens separate the images; every patch of an
 // image attends to every patch of the same image).
-#include "common.h"
+#include "attn_rows.h"
 
 // ---------------------------------------------------------------------------
 // LayerNorm over rows: y = (x - mean) * rsqrt(var + eps) * w + b, fp32 math, fp16 out
@@ -318,21 +318,25 @@ extern "C" int omni_vision_rope(void* qkv, int ld, int S, int n_heads, int head_
 // and every query t of segment [cu[s], cu[s+1]), out[t] = softmax(q_t K^T * scale) V over
 // the keys of the same segment.
 //
-// One workgroup (4 waves) owns 64 consecutive queries of one segment and one head; each
-// wave 16 of them.  K and V tiles of 64 keys are staged in LDS once for the 4 waves
-// (double buffered, the next tile's loads in flight while the current one is used).  The
-// MFMA structure is the decode / prefill kernels': S^T[16 keys x 16 queries] = K . Q^T
-// (k = 96: dims 80..95 are zero in both operands), online softmax in fp32 (exp2),
-// O[16 queries x 80] += P . V with V read back through the transposing LDS reads.
+// The 32-row tiles of attn_rows.h at 80 dims: 5 steps of 16 dims for the scores (nothing
+// padded) and three 32-dim output blocks, the third's upper 16 rows computed from whatever
+// follows a V row in LDS and never stored.  A workgroup owns 32 R consecutive queries of one
+// segment and one head, its key tiles dealt to S groups of R waves whose states merge in LDS.
+// K and V rows stay 160 bytes apart: the score operand's 16 rows x 16 bytes then repeat their
+// banks every 8 rows, which a chunk swizzle by (row / 8) % 2 undoes, and the transposed V
+// reads share banks in one row pair of four.
 // The workgroups of one head are contiguous in the XCD-aware order, so that a head's K
 // and V are read into one XCD's L2.
+// MI355X, us per launch of 16 heads, 64 rows in 4 key groups / 128 rows in 2, then 16-row
+// tiles: 1024 patches 14.2 / 17.5, 21.1; 600 10.0 / 12.7, 14.0; 500 + 260 + 700 19.2 / 14.7,
+// 27.5; 2048 44.4 / 33.5, 71.4; 2852 + 1020 95.4 / 80.9 (580 TFLOP/s), 161.4.  128 rows read
+// each staged tile twice as often and halve its traffic, but make half the workgroups: 64 rows
+// while those fit one round of the CUs.  (One key group of 128 rows is 3-7 % faster on the
+// large images and its error against 64 bits 1.6 % larger than the 16-row tiles': not used.)
 // ---------------------------------------------------------------------------
 #define VA_HD 80
-#define VA_KT 64       // keys per staged tile
-#define VA_KSTR 104    // LDS halfs per K row: 80 dims, 16 zeros (dims 80..95), 8 pad
-#define VA_VSTR 88     // LDS halfs per V row
 #define VA_CPR 10      // 16-byte chunks per 80-dim row
-#define VA_NLD 5       // tile chunks per thread: 2 * 64 * 10 / 256
+#define VA_ROWB 160    // bytes per LDS row
 
 struct VitAttnArgs {
   const half_t* qkv;   // rows [S][ld]: q heads | k heads | v heads, head_dim 80
@@ -342,205 +346,207 @@ struct VitAttnArgs {
   int ntiles, nh, S;
   half_t* out;         // [S][ldo], head h at column 80 h
   int ldo;
-  float scale_log2;
+  float scale_log2;    // > 0
+  int negate;          // the scale was negative: its sign goes to q
 };
 
-// KH key halves: with KH = 2 the workgroup has 8 waves; waves 4 h .. 4 h + 3 take the
-// queries of waves 0 .. 3 against the h-th half of the segment's key tiles (each half with
-// its own double-buffered tiles), and the two halves' softmax states are merged through
-// LDS at the end - twice the waves per CU on the same queries.
-template <int KH>
-__global__ __launch_bounds__(256 * KH, 1) void vit_attn_kernel(VitAttnArgs a) {
-#pragma clang fp contract(off)
-  __shared__ __attribute__((aligned(16))) half_t ks_lds[KH][2][VA_KT * VA_KSTR];
-  __shared__ __attribute__((aligned(16))) half_t vs_lds[KH][2][VA_KT * VA_VSTR];
+// ALIGNED: qkv and out on 16-byte boundaries, ldo a multiple of 8 (tiles straight to LDS,
+// 16-byte stores); otherwise staged through registers and stored by element.
+template <int R, int S, int KT, bool ALIGNED>
+__global__ __launch_bounds__(64 * R * S, 2) void vit_attn_kernel(VitAttnArgs a) {
+  constexpr int NB = KT / 32;
+  constexpr int TB = KT * VA_ROWB;                   // bytes of a K (or V) tile
+  constexpr int NI = 2 * KT * VA_CPR / 64;           // 1 KB pieces of a K + V tile
+  constexpr int NW = (NI + R - 1) / R;               // pieces per wave
+  constexpr int NBUF = 2;
+  static_assert(2 * KT * VA_CPR % 64 == 0 && TB % 1024 == 0, "tiles are whole 1 KB pieces");
+  constexpr int MB = R * S * 40 * 64 * 4;            // the merge's outputs
+  constexpr int LB = S * NBUF * 2 * TB + 64;         // + what the last row's third block reads
+  __shared__ __attribute__((aligned(16))) char smem[LB > MB ? LB : MB];
+  __shared__ float ml_lds[S][R][2][32];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int kh = wave >> 2;                     // key half
-  const int qw = wave & 3;                      // query block of 16
-  const int ht = tid & 255;                     // thread index within the half
-  const int q16 = lane >> 4, c16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave / R;                          // key group
+  const int rt = wave - grp * R;                     // row tile
+  const int l32 = lane & 31, hf = lane >> 5;
   const int L = xcd_logical_block(blockIdx.x, gridDim.x);
   const int h = L / a.ntiles, tile = L - h * a.ntiles;
   const int q0 = a.tiles[2 * tile], seg = a.tiles[2 * tile + 1];
   const int beg = max(a.cu[seg], 0), end = min(a.cu[seg + 1], a.S);
-  if (q0 < beg || q0 >= end) return;            // malformed table entry: nothing to do
-  const half8_t z8 = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};
-  // this half's key range, in whole tiles: half 0 takes the first ceil(n/2) tiles
-  const int ntile = (end - beg + VA_KT - 1) / VA_KT;
-  const int nt0 = (ntile + KH - 1) / KH;
-  const int kbeg = beg + (kh == 0 ? 0 : nt0 * VA_KT);
-  const int kend = kh == 0 && KH > 1 ? min(end, beg + nt0 * VA_KT) : end;
-  const int my_nt = kend > kbeg ? (kend - kbeg + VA_KT - 1) / VA_KT : 0;
+  if (q0 < beg || q0 >= end) return;                 // malformed table entry: nothing to do
+  const int nrows = min(end - q0, 32 * R);
+  const bool rows_here = 32 * rt < nrows;
+  const int row = min(32 * rt + l32, nrows - 1);
 
-  // the K tiles' dims 80..95 are zero for the whole kernel (tile stores never touch them)
-  for (int i = tid; i < KH * 2 * VA_KT * 2; i += 256 * KH) {
-    const int hb_ = i / (2 * VA_KT * 2), r1 = i - hb_ * (2 * VA_KT * 2);
-    const int bsel = r1 / (VA_KT * 2), rem = r1 - bsel * (VA_KT * 2);
-    *(half8_t*)(&ks_lds[hb_][bsel][(rem >> 1) * VA_KSTR + VA_HD + 8 * (rem & 1)]) = z8;
-  }
-
-  // this wave's query rows q0 + 16 qw + c16 (past the segment: its last row, not stored)
-  const int qrow = min(q0 + 16 * qw + c16, end - 1);
-  const half_t* qp = a.qkv + (int64_t)qrow * a.ld + h * VA_HD;
-  half8_t qf[3];
-  qf[0] = *(const half8_t*)(qp + 8 * q16);
-  qf[1] = *(const half8_t*)(qp + 32 + 8 * q16);
-  qf[2] = *(const half8_t*)(qp + 64 + 8 * (q16 & 1));
-  if (q16 >= 2) qf[2] = z8;                     // dims 80..95
-
-  // tile chunk u of this thread: index i = ht + 256 u; i < 640 is K (row i / 10, chunk
-  // i % 10), the rest V
-  int trow[VA_NLD], tsrc[VA_NLD], tdst[VA_NLD];
-  bool tv[VA_NLD];
+  half8_t qf[5];
+  {
+    const half_t* qp = a.qkv + (int64_t)(q0 + row) * a.ld + h * VA_HD + 8 * hf;
 #pragma unroll
-  for (int u = 0; u < VA_NLD; ++u) {
-    const int i = ht + 256 * u;
-    tv[u] = i >= VA_KT * VA_CPR;
-    const int j = tv[u] ? i - VA_KT * VA_CPR : i;
-    trow[u] = j / VA_CPR;
-    const int ch = j - trow[u] * VA_CPR;
-    tsrc[u] = (tv[u] ? 2 : 1) * a.nh * VA_HD + h * VA_HD + ch * 8;
-    tdst[u] = tv[u] ? trow[u] * VA_VSTR + ch * 8 : trow[u] * VA_KSTR + ch * 8;
-  }
-  half8_t tr[VA_NLD];
-  const int tok_hi = max(kend, kbeg + 1) - 1;   // a half without tiles re-reads one row
-  auto load_tile = [&](int kb) {
-#pragma unroll
-    for (int u = 0; u < VA_NLD; ++u) {
-      const int tok = min(min(kb + trow[u], tok_hi), a.S - 1);
-      tr[u] = *(const half8_t*)(a.qkv + (int64_t)tok * a.ld + tsrc[u]);
+    for (int ks = 0; ks < 5; ++ks) {
+      qf[ks] = *(const half8_t*)(qp + 16 * ks);
+      if (a.negate) qf[ks] = -qf[ks];
     }
-  };
-  auto store_tile = [&](int b) {
+  }
+
+  const int ntile = (end - beg + KT - 1) / KT;
+  const int steps = (ntile + S - 1) / S;
+  const int tbeg = grp * steps;
+  const int nt = min(steps, ntile - tbeg);           // may be <= 0
+
+  // piece J of a tile (J < NI / 2: K, else V): chunk c = 64 (J mod NI / 2) + lane is key
+  // c / 10, 16-byte chunk c % 10, the K chunks swizzled in the source address
+  uint32_t psrc[NW];
+  int prow[NW];
 #pragma unroll
-    for (int u = 0; u < VA_NLD; ++u) {
-      half_t* dst = tv[u] ? &vs_lds[kh][b][tdst[u]] : &ks_lds[kh][b][tdst[u]];
-      *(half8_t*)dst = tr[u];
+  for (int i = 0; i < NW; ++i) {
+    const int J = rt + R * i;
+    const bool is_v = J >= NI / 2;
+    const int c = 64 * (is_v ? J - NI / 2 : J) + lane;
+    prow[i] = c / VA_CPR;
+    const int ch = c - prow[i] * VA_CPR;
+    psrc[i] = (is_v ? 2u : 1u) * a.nh * (VA_HD * 2) + 16 * (is_v ? ch : ch ^ ((prow[i] >> 3) & 1));
+  }
+  const half_t* hbase = a.qkv + h * VA_HD;
+  auto stage = [&](int kb, char* dst) {
+    const half_t* src = hbase + (int64_t)kb * a.ld;
+    const int last = end - 1 - kb;                   // the last tile repeats the last key
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const int J = rt + R * i;
+      if (NI % R && J >= NI) continue;
+      const uint32_t off = (uint32_t)min(prow[i], last) * (uint32_t)a.ld * 2 + psrc[i];
+      if constexpr (ALIGNED)
+        dma16(src, off, __builtin_amdgcn_readfirstlane(lds_offset(dst)) + 1024 * J);
+      else
+        *(half8_t*)(dst + 1024 * J + 16 * lane) = *(const half8_t*)((const char*)src + off);
     }
   };
 
   float m_run = -INFINITY, l_run = 0.f;
-  f32x4 o_acc[5];
+  f32x16 o[3];
 #pragma unroll
-  for (int i = 0; i < 5; ++i) o_acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
+  const int koff = l32 * VA_ROWB + ((hf ^ ((l32 >> 3) & 1)) << 4);
+  const int i16 = lane & 15;
+  const int voff = (4 * hf + (i16 >> 2)) * VA_ROWB + ((lane >> 4) & 1) * 32 + (i16 & 3) * 8;
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-  // Double buffer per half: tile n is staged in buffer n & 1; the barrier after staging
-  // tile n also means every wave has finished reading that buffer's previous tile (n - 2).
-  // Both halves run the larger half's tile count so that every wave meets every barrier.
-  const int nt_all = nt0;                       // the first half is never the smaller
-  int b = 0;
-  load_tile(kbeg);
-  for (int it = 0; it < nt_all; ++it, b ^= 1) {
-    const int kb = kbeg + it * VA_KT;
-    store_tile(b);
-    __syncthreads();
-    if (it + 1 < my_nt) load_tile(kb + VA_KT);
-    if (it >= my_nt) continue;                  // this half is done (barriers still met)
-    const half_t* kt = ks_lds[kh][b];
-    const half_t* vt = vs_lds[kh][b];
+  char* gbuf = smem + grp * NBUF * 2 * TB;
+  if (nt > 0) stage(beg + tbeg * KT, gbuf);
+  // Q has landed (the compiler would otherwise count its loads as outstanding in the loop)
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  for (int it = 0; it < steps; ++it) {
+    const char* kt = gbuf + (it & 1) * 2 * TB;
+    const char* vt = kt + TB;
+    const int kb = beg + (tbeg + it) * KT;
+    vm_wait();             // this wave's pieces of tile it have landed; so, past the barrier,
+    lds_barrier();         // have the others', and tile it - 1's buffer is free
+    if (it + 1 < nt) stage(kb + KT, gbuf + ((it + 1) & 1) * 2 * TB);
+    if (it >= nt || !rows_here) continue;
+    f32x16 s[NB];
 #pragma unroll
-    for (int hb = 0; hb < 2; ++hb) {             // 32-key halves of the tile
-      const int k0 = kb + 32 * hb;
-      if (k0 >= kend) break;
-      f32x4 sacc[2];
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 16; ++i) s[b][i] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < 3; ++ks) {
-          const half8_t kf = *(const half8_t*)(kt + (32 * hb + 16 * j + c16) * VA_KSTR + 32 * ks + 8 * q16);
-          acc = mfma16x16x32(kf, qf[ks], acc);
-        }
-        sacc[j] = acc;
+    for (int ks = 0; ks < 5; ++ks)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        s[b] = mfma32x32x16(*(const half8_t*)(kt + 32 * VA_ROWB * b + koff + 32 * ks), qf[ks], s[b]);
+    if (kb + KT > end) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (kb + 32 * b + 8 * (i >> 2) + 4 * hf + (i & 3) >= end) s[b][i] = -INFINITY;
+    }
+    half8_t p[2 * NB];
+    softmax32<NB, 3>(s, a.scale_log2, m_run, l_run, o, p);
+#pragma unroll
+    for (int t = 0; t < 2 * NB; ++t)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const char* vp = vt + 16 * VA_ROWB * t + voff + 64 * d;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)vp);
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 8 * VA_ROWB));
+        const half4_t a0 = __builtin_bit_cast(half4_t, lo), a1 = __builtin_bit_cast(half4_t, hi);
+        o[d] = mfma32x32x16((half8_t){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]},
+                            p[t], o[d]);
       }
-      // lane holds scores of keys k0 + 16 j + 4 q16 + i for query c16
-      float sc[8];
-      float mblk = -INFINITY;
+  }
+
+  // The 10 output quads (lane half hf: dims 8 quad + 4 hf .. + 3), merged over the groups;
+  // group g finishes quad pairs g, g + S, ..
+  {
+    float x, y;
+    half_pair(l_run, x, y);
+    l_run = x + y;
+  }
+  float* om = (float*)smem;
+  __syncthreads();
+  if (rows_here) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = k0 + 16 * j + 4 * q16 + i;
-          const float s = key < kend ? sacc[j][i] * a.scale_log2 : -INFINITY;
-          sc[4 * j + i] = s;
-          mblk = fmaxf(mblk, s);
-        }
-      mblk = fmaxf(mblk, __shfl_xor(mblk, 16, 64));
-      mblk = fmaxf(mblk, __shfl_xor(mblk, 32, 64));
-      const float m_new = fmaxf(m_run, mblk);      // finite: key k0 < kend is visible
-      const float alpha = exp2f(m_run - m_new);
-      m_run = m_new;
-      half8_t pa;
-      float psum = 0.f;
-#pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8) {
-        const float p = exp2f(sc[s8] - m_new);
-        psum += p;
-        pa[s8] = (half_t)p;
-      }
-      l_run = l_run * alpha + psum;
-      float al[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) al[i] = __shfl(alpha, 4 * q16 + i, 64);
-#pragma unroll
-      for (int dt = 0; dt < 5; ++dt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o_acc[dt][i] *= al[i];
-#pragma unroll
-      for (int dt = 0; dt < 5; ++dt) {
-        const half8_t vb = lds_read_b_tr16(vt + 32 * hb * VA_VSTR + dt * 16, VA_VSTR, q16, c16);
-        o_acc[dt] = mfma16x16x32(pa, vb, o_acc[dt]);
-      }
+    for (int q = 0; q < 10; ++q)
+      *(float4*)(om + (((grp * R + rt) * 10 + q) * 64 + lane) * 4) =
+          make_float4(o[q >> 2][4 * (q & 3)], o[q >> 2][4 * (q & 3) + 1], o[q >> 2][4 * (q & 3) + 2],
+                      o[q >> 2][4 * (q & 3) + 3]);
+    if (hf == 0) {
+      ml_lds[grp][rt][0][l32] = m_run;
+      ml_lds[grp][rt][1][l32] = l_run;
     }
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
-  // per query row 4 q16 + i of this lane: the half's running max and sum
-  float mi[4], li[4];
+  __syncthreads();
+  if (!rows_here) return;
+  float M = ml_lds[0][rt][0][l32];                   // the first group is never empty
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    mi[i] = __shfl(m_run, 4 * q16 + i, 64);
-    li[i] = __shfl(l_run, 4 * q16 + i, 64);
+  for (int s = 1; s < S; ++s) M = fmaxf(M, ml_lds[s][rt][0][l32]);
+  float f[S], den = 0.f;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    f[s] = __builtin_amdgcn_exp2f(ml_lds[s][rt][0][l32] - M);
+    den += ml_lds[s][rt][1][l32] * f[s];
   }
-  if constexpr (KH == 2) {
-    // merge: the second half hands its (max, sum, O) to the first through LDS (the tile
-    // buffers are free once every wave is past the loop)
-    __syncthreads();
-    float* xch = (float*)&ks_lds[0][0][0];      // [4 query waves][64 lanes][4 m + 4 l + 20 O]
-    float* my = xch + (qw * 64 + lane) * 28;
-    if (kh == 1) {
+  const float inv = 1.0f / den;
+  half_t* op = a.out + (int64_t)(q0 + row) * a.ldo + h * VA_HD;
+  const bool mine = 32 * rt + l32 < nrows;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        my[i] = mi[i];
-        my[4 + i] = li[i];
+  for (int k = 0; k < 5; ++k) {
+    if (k % S != grp) continue;
+    unsigned w[2][2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int q = 2 * k + e;
+      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const float4 v = *(const float4*)(om + (((s * R + rt) * 10 + q) * 64 + lane) * 4);
+        acc.x = fmaf(v.x, f[s], acc.x);
+        acc.y = fmaf(v.y, f[s], acc.y);
+        acc.z = fmaf(v.z, f[s], acc.z);
+        acc.w = fmaf(v.w, f[s], acc.w);
       }
-#pragma unroll
-      for (int dt = 0; dt < 5; ++dt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) my[8 + 4 * dt + i] = o_acc[dt][i];
+      const half2_t c0 = {(half_t)(acc.x * inv), (half_t)(acc.y * inv)};
+      const half2_t c1 = {(half_t)(acc.z * inv), (half_t)(acc.w * inv)};
+      w[e][0] = __builtin_bit_cast(unsigned, c0);
+      w[e][1] = __builtin_bit_cast(unsigned, c1);
     }
-    __syncthreads();
-    if (kh == 1) return;
+    // exchanged between the lane halves: half 0 has all 8 dims of quad 2 k, half 1 of 2 k + 1
+    const auto r0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+    const auto r1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+    const u32x4 st = {r0[0], r1[0], r0[1], r1[1]};
+    if (mine) {
+      half_t* dp = op + 8 * (2 * k + hf);
+      if constexpr (ALIGNED) {
+        *(u32x4*)dp = st;
+      } else {
+        const half8_t hv = __builtin_bit_cast(half8_t, st);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float m1 = my[i], l1 = my[4 + i];
-      const float m = fmaxf(mi[i], m1);         // finite: the first half is never empty
-      const float f0 = exp2f(mi[i] - m), f1 = exp2f(m1 - m);   // m1 = -inf -> 0
-      li[i] = li[i] * f0 + l1 * f1;
-#pragma unroll
-      for (int dt = 0; dt < 5; ++dt) o_acc[dt][i] = o_acc[dt][i] * f0 + my[8 + 4 * dt + i] * f1;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int t = q0 + 16 * qw + 4 * q16 + i;
-    if (t < end && t < q0 + 64) {
-      half_t* op = a.out + (int64_t)t * a.ldo + h * VA_HD;
-      const float inv = 1.0f / li[i];
-#pragma unroll
-      for (int dt = 0; dt < 5; ++dt) op[dt * 16 + c16] = (half_t)(o_acc[dt][i] * inv);
+        for (int e = 0; e < 8; ++e) dp[e] = hv[e];
+      }
     }
   }
 }
@@ -548,11 +554,12 @@ __global__ __launch_bounds__(256 * KH, 1) void vit_attn_kernel(VitAttnArgs a) {
 // Non-causal attention within segments over the qkv rows (q | k | v heads, head_dim 80,
 // row stride ld), already rotated.  cu int32 [nseg + 1] (cu[0] = 0, increasing, cu[nseg]
 // = S); tiles int32 [ntiles][2] = (first query, segment) covering every segment in steps
-// of 64 queries; out fp16 [S][ldo] (head h at column 80 h).
-extern "C" int omni_vit_attention(const void* qkv, int ld, int S, int n_heads, int head_dim,
-                                  const int* cu_seqlens, const int* tiles, int ntiles, void* out,
-                                  int ldo, float scale, void* stream) {
+// of `rows` = 64 or 128 queries; out fp16 [S][ldo] (head h at column 80 h).
+extern "C" int omni_vit_attention_rows(const void* qkv, int ld, int S, int n_heads, int head_dim,
+                                       const int* cu_seqlens, const int* tiles, int ntiles,
+                                       void* out, int ldo, float scale, int rows, void* stream) {
   if (S < 0 || n_heads <= 0 || ntiles < 0) return OMNI_EINVAL;
+  if (rows != 64 && rows != 128) return OMNI_EINVAL;
   if (head_dim != VA_HD) return OMNI_EUNSUPPORTED;
   if (S == 0 || ntiles == 0) return OMNI_OK;
   if (!qkv || !cu_seqlens || !tiles || !out) return OMNI_EINVAL;
@@ -569,8 +576,27 @@ extern "C" int omni_vit_attention(const void* qkv, int ld, int S, int n_heads, i
   a.S = S;
   a.out = (half_t*)out;
   a.ldo = ldo;
-  a.scale_log2 = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL(vit_attn_kernel<2>, dim3((unsigned)grid), dim3(512), 0, (hipStream_t)stream, a);
+  a.scale_log2 = fabsf(scale) * 1.4426950408889634f;
+  a.negate = scale < 0.f;
+  const bool al = (((uintptr_t)qkv | (uintptr_t)out) & 15) == 0 && (ldo & 7) == 0;
+  const dim3 gd((unsigned)grid);
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 bd(512);
+  if (rows == 128) {
+    if (al) hipLaunchKernelGGL((vit_attn_kernel<4, 2, 64, true>), gd, bd, 0, st, a);
+    else hipLaunchKernelGGL((vit_attn_kernel<4, 2, 64, false>), gd, bd, 0, st, a);
+  } else {
+    if (al) hipLaunchKernelGGL((vit_attn_kernel<2, 4, 32, true>), gd, bd, 0, st, a);
+    else hipLaunchKernelGGL((vit_attn_kernel<2, 4, 32, false>), gd, bd, 0, st, a);
+  }
   OMNI_CHECK_LAUNCH();
   return OMNI_OK;
+}
+
+// omni_vit_attention_rows with tiles of 64 queries.
+extern "C" int omni_vit_attention(const void* qkv, int ld, int S, int n_heads, int head_dim,
+                                  const int* cu_seqlens, const int* tiles, int ntiles, void* out,
+                                  int ldo, float scale, void* stream) {
+  return omni_vit_attention_rows(qkv, ld, S, n_heads, head_dim, cu_seqlens, tiles, ntiles, out,
+                                 ldo, scale, 64, stream);
 }

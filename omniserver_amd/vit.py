@@ -23,11 +23,12 @@ from typing import Dict, List, Sequence, Tuple
 import torch
 
 from ._lib import call, lib, ptr, require_cuda, stream
+from .attention import num_cus
 from .hostio import to_device
 
 EPI_STORE, EPI_QGELU, EPI_GELU, EPI_RESID = 0, 4, 5, 6
 EPI_PARTIAL = 2
-_QT = 64     # queries per attention workgroup (the kernel's tile)
+_QT = 64     # queries per attention workgroup (the kernel's smaller tile; the other is 128)
 
 
 @dataclass
@@ -104,10 +105,10 @@ def cu_seqlens(grid_thw) -> torch.Tensor:
     return torch.tensor(cu, dtype=torch.int32)
 
 
-def query_tiles(cu: torch.Tensor) -> torch.Tensor:
-    """int32 [ntiles, 2] = (first query, segment): every segment in steps of 64 queries."""
+def query_tiles(cu: torch.Tensor, step: int = _QT) -> torch.Tensor:
+    """int32 [ntiles, 2] = (first query, segment): every segment in steps of ``step`` queries."""
     c = cu.tolist()
-    rows = [(q, s) for s in range(len(c) - 1) for q in range(c[s], c[s + 1], _QT)]
+    rows = [(q, s) for s in range(len(c) - 1) for q in range(c[s], c[s + 1], step)]
     return torch.tensor(rows, dtype=torch.int32).view(-1, 2)
 
 
@@ -151,13 +152,26 @@ def vision_rope_(qkv: torch.Tensor, n_heads: int, head_dim: int, pos_hw: torch.T
 
 
 def vit_attention_out(qkv: torch.Tensor, n_heads: int, head_dim: int, cu: torch.Tensor,
-                      tiles: torch.Tensor, scale: float, out: torch.Tensor) -> torch.Tensor:
-    """Non-causal attention within the segments cu (int32, device) of the rotated qkv rows."""
+                      tiles: torch.Tensor, scale: float, out: torch.Tensor,
+                      step: int = _QT) -> torch.Tensor:
+    """Non-causal attention within the segments cu (int32, device) of the rotated qkv rows;
+    ``step``: the query_tiles step (64 or 128) the tiles were made with."""
     require_cuda(qkv, out, dtype=torch.float16)
     require_cuda(cu, tiles, dtype=torch.int32)
-    call("omni_vit_attention", ptr(qkv), qkv.stride(0), qkv.shape[0], n_heads, head_dim, ptr(cu),
-         ptr(tiles), tiles.shape[0], ptr(out), out.stride(0), float(scale), stream())
+    call("omni_vit_attention_rows", ptr(qkv), qkv.stride(0), qkv.shape[0], n_heads, head_dim,
+         ptr(cu), ptr(tiles), tiles.shape[0], ptr(out), out.stride(0), float(scale), step,
+         stream())
     return out
+
+
+def attention_step(cu: torch.Tensor, n_heads: int, device) -> int:
+    """Queries per attention workgroup for the segments cu (host): 64, its keys in 4 groups,
+    while those workgroups fit one round of the CUs (1024 patches: 14.2 us against 17.5), else
+    128 in 2 groups, which stage each key tile for twice the rows (2048 patches: 33.5 against
+    44.4)."""
+    c = cu.tolist()
+    tiles = sum(-(-(b - a) // _QT) for a, b in zip(c, c[1:]))
+    return _QT if tiles * n_heads <= num_cus(device) else 2 * _QT
 
 
 class VisionLinear:
@@ -295,9 +309,10 @@ class Qwen2VIT:
         m2 = cfg.spatial_merge_size ** 2
         pos = to_device(rot_pos_ids(grids, cfg.spatial_merge_size), torch.int32, dev)
         cu_h = cu_seqlens(grids)
-        tiles = to_device(query_tiles(cu_h), torch.int32, dev)
         cu = to_device(cu_h, torch.int32, dev)
         D, nh, hd = cfg.embed_dim, cfg.n_heads, cfg.head_dim
+        step = attention_step(cu_h, nh, dev)
+        tiles = to_device(query_tiles(cu_h, step), torch.int32, dev)
         mk = lambda *s: torch.empty(*s, device=dev, dtype=torch.float16)
         x, h, att = mk(S, D), mk(S, D), mk(S, D)
         qkv, f = mk(S, 3 * D), mk(S, cfg.mlp_dim)
@@ -317,7 +332,7 @@ class Qwen2VIT:
                 layer_norm_partials_out(parts, pend[0], pend[1], x, blk.n1w, blk.n1b, cfg.eps, h)
             blk.qkv.out(h, qkv)
             vision_rope_(qkv, nh, hd, pos, self.inv_freq)
-            vit_attention_out(qkv, nh, hd, cu, tiles, scale, att)
+            vit_attention_out(qkv, nh, hd, cu, tiles, scale, att, step)
             _, sp = blk.proj.out_partial(att, parts)
             layer_norm_partials_out(parts, sp, blk.proj.bias, x, blk.n2w, blk.n2b, cfg.eps, h)
             blk.fc1.out(h, f, EPI_QGELU)

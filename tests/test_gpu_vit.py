@@ -129,6 +129,32 @@ def test_gemm_epilogues(gpu, M, N, K, epi, has_bias, path, tile_rows, ksplit):
     assert (d <= tol).all(), d.max().item()
 
 
+@pytest.mark.parametrize("step", [64, 128])
+@pytest.mark.parametrize("segs", [[1], [31, 33], [64, 128, 65], [129, 4, 500]])
+@pytest.mark.parametrize("scale,off", [(80 ** -0.5, 0), (-0.2, 0), (80 ** -0.5, 4)])
+def test_vit_attention_tiles(gpu, segs, step, scale, off):
+    """Both workgroup shapes of the segmented attention against float64: segments on both
+    sides of the 32 / 64-key tiles and of the row tiles, fewer key tiles than key groups, a
+    negative scale (its sign rides on q) and a qkv base 8 bytes off the 16-byte boundary (the
+    register-staged form).  Tolerance: the fp16 rounding of P and of the output, V ~ N(0, 1)."""
+    from omniserver_amd import vit
+    nh, hd = 3, 80
+    S = sum(segs)
+    say(f"vit_attention step={step} segs={segs} scale={scale:.3f} off={off}")
+    buf = torch.empty(S * 3 * nh * hd + 8, dtype=torch.float16)
+    buf.copy_(f16((buf.numel(),), 10))
+    qkv = buf.to(gpu)[off:off + S * 3 * nh * hd].view(S, 3 * nh * hd)
+    cu = torch.tensor([sum(segs[:i]) for i in range(len(segs) + 1)], dtype=torch.int32)
+    out = torch.full((S, nh * hd), float("nan"), device=gpu, dtype=torch.float16)
+    vit.vit_attention_out(qkv, nh, hd, cu.to(gpu), vit.query_tiles(cu, step).to(gpu), scale, out, step)
+    q, k, v = qkv.cpu().double().view(S, 3, nh, hd).unbind(1)
+    for a, b in zip(cu.tolist(), cu.tolist()[1:]):
+        for h in range(nh):
+            want = torch.softmax(q[a:b, h] @ k[a:b, h].t() * scale, -1) @ v[a:b, h]
+            d = (out[a:b, h * hd:(h + 1) * hd].cpu().double() - want).abs().max().item()
+            assert d <= 4e-3, (a, h, d)
+
+
 def _tower(gpu, depth, seed):
     from omniserver_amd import synth, vit
     cfg = vit.VisionConfig(depth=depth)
