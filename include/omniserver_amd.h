@@ -81,6 +81,13 @@ int omni_silu_mul(const void* gate_up, void* out, int rows, int n, void* stream)
  * bf16, model/qwen2_llm.py:127-131): out bf16 [rows, n], fp32 math, bf16 stores (RNE). */
 int omni_silu_mul_bf16(const void* gate_up, void* out, int rows, int n, void* stream);
 
+/* silu_mul (bf16 = 1: on bf16) that also leaves partial maxima of |out| in part, for
+ * omni_fp8_quant_tensor_parts (FP8Linear's per-tensor scale, kernels/fp8_linear.py:40-41):
+ * omni_silu_mul_amax_parts(rows, n) floats. */
+int omni_silu_mul_amax(const void* gate_up, void* out, float* part, int rows, int n, int bf16,
+                       void* stream);
+int omni_silu_mul_amax_parts(int rows, int n);
+
 /* ---------------------------------------------------------------- rope + KV pool */
 
 /* apply_mrope (model/qwen2_llm.py:59-72) in place on the q and k heads of qkv rows
@@ -447,6 +454,10 @@ int omni_fp8_quant_weight_rows(const void* w, int ldw, void* wq, float* scale, i
 int omni_fp8_quant_tensor(const void* x, int ldx, void* q, float* scale, float* work,
                           int rows, int K, int bf16, void* stream);
 int omni_fp8_quant_tensor_work(int rows);
+
+/* omni_fp8_quant_tensor's second launch, on nparts partial maxima of |x| already in part. */
+int omni_fp8_quant_tensor_parts(const void* x, int ldx, void* q, float* scale, const float* part,
+                                int nparts, int rows, int K, int bf16, void* stream);
 
 /* FP8Linear.forward / forward_prequant (kernels/fp8_linear.py:99-126): the product
  * v[m, n] = (sum_k xq[m,k] wq[n,k]) * sa[m] * sw[n] (fp32 accumulation, as

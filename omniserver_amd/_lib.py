@@ -34,6 +34,8 @@ SIGNATURES = {
     "omni_embedding": [_P, _P, _I, _I64, _P, _I, _I, _P],
     "omni_silu_mul": [_P, _P, _I, _I, _P],
     "omni_silu_mul_bf16": [_P, _P, _I, _I, _P],
+    "omni_silu_mul_amax": [_P, _P, _P, _I, _I, _I, _P],
+    "omni_silu_mul_amax_parts": [_I, _I],
     "omni_mrope_kv_write": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                             _I, _I, _I, _I, _P],
     "omni_mrope_kv_write_partials": [_P, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P,
@@ -47,6 +49,7 @@ SIGNATURES = {
     "omni_fp8_quant_weight_rows": [_P, _I, _P, _P, _I, _I, _P],
     "omni_fp8_quant_tensor": [_P, _I, _P, _P, _P, _I, _I, _I, _P],
     "omni_fp8_quant_tensor_work": [_I],
+    "omni_fp8_quant_tensor_parts": [_P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
     "omni_fp8_gemm": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "omni_fp8_gemm_plan": [_I, _I, _I, ctypes.POINTER(_I)],
     "omni_w4a16_gemm_attn": [_P, _I, _I, _I, _P, _P, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I,

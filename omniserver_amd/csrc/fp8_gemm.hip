@@ -493,26 +493,28 @@ __global__ __launch_bounds__(128 * WM, 1) void fp8_gemm_pipe_kernel(Fp8GemmArgs 
 // quarter of the CUs idle.
 #define F8B_T 256
 
-// Output bits of one product value v = acc * sa * sw: bf16(v), then either that bf16 plus
-// bf16(bias) as a bf16 add (FP8_OUT_BF16: forward_prequant, out + bias.to(bf16)) or the
-// bf16 rounded to fp16 plus the fp16 bias as an fp16 add (FP8_OUT_F16_VIA_BF16: the
-// row-wise forward).  A zero bias is the identity in both (x + 0 rounds to x).  The
-// per-tensor form (FP8_OUT_F16) does not run here (omni_fp8_gemm sends it to the 256 x 128
-// kernel, which has all three forms).
-template <bool OUT_BF16>
-__device__ __forceinline__ uint32_t fp8_out_bits(float v, half_t bias) {
-  const uint32_t b = f32_to_bf16_bits(v);
-  const float bf = __builtin_bit_cast(float, b << 16);
-  if (OUT_BF16) return f32_to_bf16_bits(bf + bf16_value((float)bias));
-  return (uint32_t)__builtin_bit_cast(uint16_t, (half_t)((float)(half_t)bf + (float)bias));
-}
-
-// fp8_out_bits of two adjacent outputs, packed (v0 low): one bf16 conversion per pair.
-template <bool OUT_BF16>
-__device__ __forceinline__ uint32_t fp8_out_bits2(float v0, float v1, half_t b0, half_t b1) {
+// Two adjacent product values v = acc * sa * sw stored, packed (v0 low), in out_mode's form:
+// bf16(v) plus bf16(bias) as a bf16 add (FP8_OUT_BF16: forward_prequant, out + bias.to(bf16)),
+// that bf16 rounded to fp16 plus the fp16 bias as an fp16 add (FP8_OUT_F16_VIA_BF16: the
+// row-wise forward) - in both a zero bias is the identity (x + 0 rounds to x), and the bf16
+// conversion is one per pair - or fp16(v) plus the fp16 bias (FP8_OUT_F16: the per-tensor
+// forward).
+template <int MODE>
+__device__ __forceinline__ uint32_t fp8_out_bits2(float v0, float v1, half_t b0, half_t b1,
+                                                  bool has_bias) {
+  if (MODE == FP8_OUT_F16) {
+    // opaque: the scale multiply and the conversion would fold into one rounding
+    asm("" : "+v"(v0), "+v"(v1));
+    half_t h0 = (half_t)v0, h1 = (half_t)v1;
+    if (has_bias) {
+      h0 = (half_t)((float)h0 + (float)b0);
+      h1 = (half_t)((float)h1 + (float)b1);
+    }
+    return (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+  }
   const uint32_t p = bf16x2_bits(v0, v1);
   const float f0 = __builtin_bit_cast(float, p << 16), f1 = __builtin_bit_cast(float, p & 0xffff0000u);
-  if (OUT_BF16) return bf16x2_bits(f0 + bf16_value((float)b0), f1 + bf16_value((float)b1));
+  if (MODE == FP8_OUT_BF16) return bf16x2_bits(f0 + bf16_value((float)b0), f1 + bf16_value((float)b1));
   const half_t h0 = (half_t)((float)(half_t)f0 + (float)b0);
   const half_t h1 = (half_t)((float)(half_t)f1 + (float)b1);
   return (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
@@ -529,7 +531,7 @@ __device__ __forceinline__ uint32_t fp8_out_bits2(float v0, float v1, half_t b0,
 // (fp8_tail_cols); such a tile loads 3 of the 4 row groups of w, reads its wave's 3 n
 // sub-tiles from 48 wn plus a fourth fragment from the slot's next 16 rows (unused), and
 // stores 3 of its 4 n sub-tiles, so both kinds share the loop's code and registers.
-template <bool OUT_BF16, int NIW, typename ReadCol>
+template <int MODE, int NIW, typename ReadCol>
 __device__ __forceinline__ void fp8_bigp_epilogue(const f32x4 (&acc)[NIW][8], uint16_t* ob, int ldo,
                                                   const float (&sm)[8], ReadCol read_col,
                                                   bool has_bias, int ni) {
@@ -549,8 +551,8 @@ __device__ __forceinline__ void fp8_bigp_epilogue(const f32x4 (&acc)[NIW][8], ui
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = (acc[i][j][q] * sm[j]) * sn_i[q];
       uint2 pk;
-      pk.x = fp8_out_bits2<OUT_BF16>(v[0], v[1], bb[0], bb[1]);
-      pk.y = fp8_out_bits2<OUT_BF16>(v[2], v[3], bb[2], bb[3]);
+      pk.x = fp8_out_bits2<MODE>(v[0], v[1], bb[0], bb[1], has_bias);
+      pk.y = fp8_out_bits2<MODE>(v[2], v[3], bb[2], bb[3], has_bias);
       *(uint2*)(ob + (16 * j * ldo + 16 * i)) = pk;
     }
   }
@@ -814,8 +816,12 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
                            ((ln & 15u) * (uint32_t)a.ldo + 4u * (ln >> 4));
       auto rc = [&](int i, f32x4& sn, u32x2& bw) { read_col(r & 1, cw, i, sn, bw); };
       const int ni = TAIL && tlc ? 3 : NIW;           // n sub-tiles stored
-      if (a.out_mode) fp8_bigp_epilogue<true, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
-      else fp8_bigp_epilogue<false, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
+      if (a.out_mode == FP8_OUT_BF16)
+        fp8_bigp_epilogue<FP8_OUT_BF16, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
+      else if (a.out_mode == FP8_OUT_F16)
+        fp8_bigp_epilogue<FP8_OUT_F16, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
+      else
+        fp8_bigp_epilogue<FP8_OUT_F16_VIA_BF16, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
     }
     m0c = m0n;
     n0c = n0n;
@@ -863,14 +869,13 @@ __global__ __launch_bounds__(256) void fp8_quant_rows_kernel(const unsigned shor
   if (S16) sc = (float)(half_t)sc;
   if (clamp_min > 0.f) sc = fmaxf(sc, clamp_min);
   if (threadIdx.x == 0) s[row] = sc;
+  const Fp8Scale d(sc);
   for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
     const u16x8 v = *(const u16x8*)(xr + k);
-    uint32_t lo = 0, hi = 0;
+    float f[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) lo |= (uint32_t)f32_to_e4m3fn(ld16f<BF16>(v[e]) / sc) << (8 * e);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) hi |= (uint32_t)f32_to_e4m3fn(ld16f<BF16>(v[4 + e]) / sc) << (8 * e);
-    *(uint2*)(q + (int64_t)row * K + k) = make_uint2(lo, hi);
+    for (int e = 0; e < 8; ++e) f[e] = ld16f<BF16>(v[e]);
+    *(uint2*)(q + (int64_t)row * K + k) = fp8_codes8<1>(f, d, [](float t) { return t; });
   }
 }
 
@@ -906,29 +911,59 @@ extern "C" int omni_fp8_quant_weight_rows(const void* w, int ldw, void* wq, floa
 // Per-tensor e4m3 quantisation (FP8Linear's default form): s = R(amax |x| / 448) and
 // q = e4m3(R(x / s)), R the input's own rounding (fp16, or bf16 for bf16 input): the
 // reference forms both with ops on the fp16 / bf16 tensor (fp8_linear.py:40-41, 87-89).
-// Two launches, no atomics: fp8_amax_kernel writes one partial maximum per workgroup
-// (rows b, b + grid, ...), fp8_quant_tensor_kernel reduces the grid's partials in every
-// workgroup and quantises the same rows, writing s into scale[r] for each of them.
+// Two launches, no atomics: fp8_amax_kernel writes one partial maximum per workgroup,
+// fp8_quant_tensor_kernel reduces the partials in every workgroup, quantises and writes s into
+// scale[r] for every row.  Both walk the 8-value chunks of all rows, the first with 256
+// workgroups of 1024 threads and 4 chunks in flight each, the second with 1024 chunks per
+// workgroup: at [8192, 8960] bf16 85 -> 31 and 230 -> 53 us (4.7 and 4.2 TB/s; a plain copy
+// moves 5.2) against one row per workgroup at a time with a division and a software
+// conversion per value.
 #define FP8_AMAX_GRID 256
+#define FP8_AMAX_NT 1024
+
+// Chunk i of rows of nc chunks, ldx elements apart: its address (dense: ldx = 8 nc).
+__device__ __forceinline__ const unsigned short* fp8_chunk(const unsigned short* x, int ldx,
+                                                           uint32_t nc, bool dense, uint64_t i) {
+  if (dense) return x + i * 8;
+  const uint64_t r = i / nc;
+  return x + r * (uint64_t)ldx + (i - r * nc) * 8;
+}
 
 template <bool BF16>
-__global__ __launch_bounds__(256) void fp8_amax_kernel(const unsigned short* __restrict__ x,
-                                                       int ldx, int rows, int K,
-                                                       float* __restrict__ part) {
-  __shared__ float red[4];
-  float amax = 0.f;
-  for (int r = blockIdx.x; r < rows; r += gridDim.x) {
-    const unsigned short* xr = x + (int64_t)r * ldx;
-    for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
-      const u16x8 v = *(const u16x8*)(xr + k);
+__device__ __forceinline__ float amax8(const u16x8& v, float amax) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(ld16f<BF16>(v[e])));
+  for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(ld16f<BF16>(v[e])));
+  return amax;
+}
+
+template <bool BF16>
+__global__ __launch_bounds__(FP8_AMAX_NT) void fp8_amax_kernel(const unsigned short* __restrict__ x,
+                                                               int ldx, int rows, int K,
+                                                               float* __restrict__ part) {
+  __shared__ float red[FP8_AMAX_NT / 64];
+  const uint32_t nc = (uint32_t)K >> 3;
+  const uint64_t total = (uint64_t)rows * nc;
+  const bool dense = ldx == K;
+  const uint64_t stride = (uint64_t)gridDim.x * FP8_AMAX_NT;
+  float amax = 0.f;
+  for (uint64_t i = (uint64_t)blockIdx.x * FP8_AMAX_NT + threadIdx.x; i < total; i += 4 * stride) {
+    u16x8 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {          // past the end: the last chunk again
+      const uint64_t j = i + u * stride;
+      v[u] = *(const u16x8*)fp8_chunk(x, ldx, nc, dense, j < total ? j : total - 1);
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) amax = amax8<BF16>(v[u], amax);
   }
   amax = wave_max(amax);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < FP8_AMAX_NT / 64; ++w) amax = fmaxf(amax, red[w]);
+    part[blockIdx.x] = amax;
+  }
 }
 
 template <bool BF16>
@@ -940,36 +975,61 @@ template <bool BF16>
 __global__ __launch_bounds__(256) void fp8_quant_tensor_kernel(const unsigned short* __restrict__ x,
                                                                int ldx, int rows, int K,
                                                                const float* __restrict__ part,
-                                                               uint8_t* __restrict__ q,
+                                                               int nparts, uint8_t* __restrict__ q,
                                                                float* __restrict__ s) {
 #pragma clang fp contract(off)
   __shared__ float red[4];
+  const uint32_t nc = (uint32_t)K >> 3;
+  const uint64_t total = (uint64_t)rows * nc;
+  const bool dense = ldx == K;
+  const uint64_t i0 = (uint64_t)blockIdx.x * 1024 + threadIdx.x;
+  u16x8 v[4];                               // requested ahead of the partial maxima
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const uint64_t j = i0 + 256 * u;
+    v[u] = *(const u16x8*)fp8_chunk(x, ldx, nc, dense, j < total ? j : total - 1);
+  }
   float amax = 0.f;
-  for (int i = threadIdx.x; i < (int)gridDim.x; i += 256) amax = fmaxf(amax, part[i]);
+  for (int i = threadIdx.x; i < nparts; i += 256) amax = fmaxf(amax, part[i]);
   amax = wave_max(amax);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   const float sc = round_in<BF16>(amax / 448.0f);
-  for (int r = blockIdx.x; r < rows; r += gridDim.x) {
-    const unsigned short* xr = x + (int64_t)r * ldx;
-    if (threadIdx.x == 0) s[r] = sc;
-    for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
-      const u16x8 v = *(const u16x8*)(xr + k);
-      uint32_t lo = 0, hi = 0;
+  const Fp8Scale d(sc);
+  for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < rows; r += (int64_t)gridDim.x * 256)
+    s[r] = sc;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        lo |= (uint32_t)f32_to_e4m3fn(round_in<BF16>(ld16f<BF16>(v[e]) / sc)) << (8 * e);
+  for (int u = 0; u < 4; ++u) {
+    const uint64_t j = i0 + 256 * u;
+    if (j >= total) break;
+    float f[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        hi |= (uint32_t)f32_to_e4m3fn(round_in<BF16>(ld16f<BF16>(v[4 + e]) / sc)) << (8 * e);
-      *(uint2*)(q + (int64_t)r * K + k) = make_uint2(lo, hi);
-    }
+    for (int e = 0; e < 8; ++e) f[e] = ld16f<BF16>(v[u][e]);
+    *(uint2*)(q + j * 8) = fp8_codes8<1>(f, d, [](float t) { return round_in<BF16>(t); });
   }
 }
 
 extern "C" int omni_fp8_quant_tensor_work(int rows) {
   return rows <= 0 ? 0 : (rows < FP8_AMAX_GRID ? rows : FP8_AMAX_GRID);
+}
+
+// The second launch alone, on nparts partial maxima of |x| that another kernel left in part
+// (omni_silu_mul_amax).
+extern "C" int omni_fp8_quant_tensor_parts(const void* x, int ldx, void* q, float* scale,
+                                           const float* part, int nparts, int rows, int K,
+                                           int bf16, void* stream) {
+  if (rows < 0 || K <= 0) return OMNI_EINVAL;
+  if ((K & 7) || ldx < K || (ldx & 7)) return OMNI_EUNSUPPORTED;
+  if (rows == 0) return OMNI_OK;
+  if (!x || !q || !scale || !part || nparts <= 0) return OMNI_EINVAL;
+  const int64_t grid = ((int64_t)rows * (K >> 3) + 1023) / 1024;
+  if (grid > 0x7fffffff) return OMNI_EUNSUPPORTED;
+  auto kern = bf16 ? fp8_quant_tensor_kernel<true> : fp8_quant_tensor_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream,
+                     (const unsigned short*)x, ldx, rows, K, part, nparts, (uint8_t*)q, scale);
+  OMNI_CHECK_LAUNCH();
+  return OMNI_OK;
 }
 
 extern "C" int omni_fp8_quant_tensor(const void* x, int ldx, void* q, float* scale, float* work,
@@ -979,23 +1039,11 @@ extern "C" int omni_fp8_quant_tensor(const void* x, int ldx, void* q, float* sca
   if (rows == 0) return OMNI_OK;
   if (!x || !q || !scale || !work) return OMNI_EINVAL;
   const int grid = omni_fp8_quant_tensor_work(rows);
-  if (bf16) {
-    hipLaunchKernelGGL(fp8_amax_kernel<true>, dim3(grid), dim3(256), 0, (hipStream_t)stream,
-                       (const unsigned short*)x, ldx, rows, K, work);
-    OMNI_CHECK_LAUNCH();
-    hipLaunchKernelGGL(fp8_quant_tensor_kernel<true>, dim3(grid), dim3(256), 0,
-                       (hipStream_t)stream, (const unsigned short*)x, ldx, rows, K, work,
-                       (uint8_t*)q, scale);
-  } else {
-    hipLaunchKernelGGL(fp8_amax_kernel<false>, dim3(grid), dim3(256), 0, (hipStream_t)stream,
-                       (const unsigned short*)x, ldx, rows, K, work);
-    OMNI_CHECK_LAUNCH();
-    hipLaunchKernelGGL(fp8_quant_tensor_kernel<false>, dim3(grid), dim3(256), 0,
-                       (hipStream_t)stream, (const unsigned short*)x, ldx, rows, K, work,
-                       (uint8_t*)q, scale);
-  }
+  auto kern = bf16 ? fp8_amax_kernel<true> : fp8_amax_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(FP8_AMAX_NT), 0, (hipStream_t)stream,
+                     (const unsigned short*)x, ldx, rows, K, work);
   OMNI_CHECK_LAUNCH();
-  return OMNI_OK;
+  return omni_fp8_quant_tensor_parts(x, ldx, q, scale, work, grid, rows, K, bf16, stream);
 }
 
 // Kernel choice by shape: the persistent big tiles (256 x 256 or 256 x 192) where a cost
@@ -1027,8 +1075,8 @@ static int fp8_tail_cols(int M, int N) {
   return (int)(nb * 256);
 }
 
-static int fp8_big_cols(int M, int N, int K, int out_mode = FP8_OUT_F16_VIA_BF16) {
-  if (K < 1024 || (M % F8B_T) || out_mode == FP8_OUT_F16) return 0;
+static int fp8_big_cols(int M, int N, int K) {
+  if (K < 1024 || (M % F8B_T)) return 0;
   const int64_t cus = num_cus();
   auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
   double best = (double)rounds((int64_t)(M / 256) * (N / F8_BT));   // pipelined tiles
@@ -1099,7 +1147,7 @@ extern "C" int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, co
   a.K = K;
   a.out_mode = out_mode;
   a.n_big = N;
-  const int bc = fp8_big_cols(M, N, K, out_mode);
+  const int bc = fp8_big_cols(M, N, K);
   if (bc) {                                       // persistent 256 x bc tiles
     if (bc == 256) a.n_big = fp8_tail_cols(M, N);
     const int64_t bt = fp8_big_items(M, N, bc);

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from ._lib import call, ptr, require_cuda, stream
+from ._lib import call, lib, ptr, require_cuda, stream
 
 
 def _rows(x: torch.Tensor) -> tuple[int, int]:
@@ -90,6 +90,23 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     n = gate_up.shape[-1] // 2
     out = torch.empty(*gate_up.shape[:-1], n, device=gate_up.device, dtype=gate_up.dtype)
     return silu_mul_out(gate_up, out)
+
+
+def silu_mul_amax(gate_up: torch.Tensor):
+    """silu_mul and fp32 partial maxima of its magnitudes (what a per-tensor FP8Linear's
+    ``amax_parts`` takes), in one launch."""
+    gate_up = gate_up.contiguous()
+    require_cuda(gate_up)
+    if gate_up.dtype not in (torch.float16, torch.bfloat16):
+        raise TypeError(f"silu_mul takes fp16 or bf16 (got {gate_up.dtype})")
+    m, n2 = _rows(gate_up)
+    n = n2 // 2
+    out = torch.empty(*gate_up.shape[:-1], n, device=gate_up.device, dtype=gate_up.dtype)
+    part = torch.empty(lib().omni_silu_mul_amax_parts(m, n), device=gate_up.device,
+                       dtype=torch.float32)
+    call("omni_silu_mul_amax", ptr(gate_up), ptr(out), ptr(part), m, n,
+         int(gate_up.dtype == torch.bfloat16), stream())
+    return out, part
 
 
 def embedding_out(ids, table, packed: bool, out):

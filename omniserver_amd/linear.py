@@ -568,10 +568,12 @@ class FP8Linear(nn.Module):
         """The reference's ``wscale``: [1, N] row-wise, a 0-dim scalar per-tensor."""
         return self.weight_scale.view(1, -1) if self.rowwise else self.weight_scale[0]
 
-    def quantize_input(self, x2d: torch.Tensor):
+    def quantize_input(self, x2d: torch.Tensor, amax_parts: torch.Tensor | None = None):
         """The forward's activation quantisation of fp16 or bf16 rows: (xq e4m3 bytes
         [M, K], scale fp32 [M, 1]) - per token (quant_fp8, fp8_linear.py:45-63) for the
-        row-wise form, one value repeated for the per-tensor form (:40-41)."""
+        row-wise form, one value repeated for the per-tensor form (:40-41).  ``amax_parts``:
+        fp32 partial maxima of |x2d| that its producer left (the per-tensor form then reads
+        x2d once)."""
         M = x2d.shape[0]
         xq = torch.empty(M, self.K, device=x2d.device, dtype=torch.uint8)
         sa = torch.empty(M, 1, device=x2d.device, dtype=torch.float32)
@@ -579,6 +581,9 @@ class FP8Linear(nn.Module):
         if self.rowwise:
             fn = "omni_fp8_quant_rows_bf16" if bf16 else "omni_fp8_quant_rows"
             call(fn, ptr(x2d), x2d.stride(0), ptr(xq), ptr(sa), M, self.K, 0.0, stream())
+        elif amax_parts is not None and amax_parts.numel():
+            call("omni_fp8_quant_tensor_parts", ptr(x2d), x2d.stride(0), ptr(xq), ptr(sa),
+                 ptr(amax_parts), amax_parts.numel(), M, self.K, int(bf16), stream())
         else:
             work = torch.empty(lib().omni_fp8_quant_tensor_work(M), device=x2d.device,
                                dtype=torch.float32)
@@ -611,16 +616,16 @@ class FP8Linear(nn.Module):
         self.gemm_out(xq2, scale.reshape(-1).contiguous().float(), out, self.OUT_BF16)
         return out.reshape(*xq.shape[:-1], self.N)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, amax_parts: torch.Tensor | None = None) -> torch.Tensor:
         """fp16 or bf16 x (the bf16 silu_mul output of the fused FP8 MLP route,
-        qwen2_llm.py:132-134) -> fp16."""
+        qwen2_llm.py:132-134) -> fp16.  ``amax_parts``: see quantize_input."""
         x2d = x.reshape(-1, self.K)
         if not x2d.is_contiguous():
             x2d = x2d.contiguous()
         require_cuda(x2d)
         if x2d.dtype not in (torch.float16, torch.bfloat16):
             raise TypeError(f"expected fp16 or bf16 activations, got {x2d.dtype}")
-        xq, sa = self.quantize_input(x2d)
+        xq, sa = self.quantize_input(x2d, amax_parts)
         out = torch.empty(x2d.shape[0], self.N, device=x.device, dtype=torch.float16)
         self.gemm_out(xq, sa, out, self.OUT_F16_VIA_BF16 if self.rowwise else self.OUT_F16)
         return out.reshape(*x.shape[:-1], self.N)

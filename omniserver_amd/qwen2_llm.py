@@ -23,7 +23,7 @@ from torch import nn
 
 from . import fused_ops as F
 from .hostio import to_device
-from .linear import F16Linear, GPTQLinear, LMHeadArgmax, _Skinny
+from .linear import F16Linear, FP8Linear, GPTQLinear, LMHeadArgmax, _Skinny
 from .synth import DecoderShape
 
 Qwen2Config = DecoderShape
@@ -102,7 +102,15 @@ class MLP(nn.Module):
             gu = self.gate_up_proj.forward_prequant(xq, scale)
         else:
             gu = self.gate_up_proj(x)
-        out = gu if getattr(self.gate_up_proj, "fuse_silu", False) else F.silu_mul(gu)
+        if getattr(self.gate_up_proj, "fuse_silu", False):
+            out = gu
+        elif (getattr(self.down_proj.forward, "__func__", None) is FP8Linear.forward
+                and not self.down_proj.rowwise and gu.numel()):
+            # a per-tensor FP8 down: its input's maximum comes out of the SiLU-mul's launch
+            out, parts = F.silu_mul_amax(gu)
+            return self.down_proj(out, parts)
+        else:
+            out = F.silu_mul(gu)
         if out.dtype != torch.float16 and not hasattr(self.down_proj, "forward_prequant"):
             out = out.to(torch.float16)
         return self.down_proj(out)

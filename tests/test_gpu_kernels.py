@@ -1222,6 +1222,114 @@ def test_fp8_quant_tensor_bit_exact(gpu, rows, K, bf16):
     assert torch.equal(q.cpu(), eq.view(torch.uint8))
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("case", ["zeros", "signs", "tiny", "nan", "inf", "strided"])
+def test_fp8_quant_edges(gpu, case, bf16):
+    """Both activation quantisers where the corrected-reciprocal division or the hardware
+    conversion could part from fp32 division and the software rounding: signed zeros, scales
+    that are zero, subnormal or out of the fast range, NaN and infinite inputs (codes compared,
+    signed zeros included), rows apart in memory.  Bit-exact against the same formulas on the
+    CPU, the sign of a NaN apart (division and rounding define none)."""
+    from omniserver_amd._lib import call, lib, ptr, stream
+    say(f"fp8 quantisation edges {case} bf16={bf16}")
+    rows, K = 5, 264
+    dt = torch.bfloat16 if bf16 else torch.float16
+    x = f16((rows, K), 160, 1.5).to(dt)
+    if case == "zeros":
+        x.zero_()
+        x[1] = -0.0
+    elif case == "signs":
+        x[:, ::3] = -0.0
+        x[2] *= 2.0 ** -13
+    elif case == "tiny":
+        x = (x.double() * 2.0 ** (-120 if bf16 else -22)).to(dt)
+    elif case == "nan":
+        x[0, 5] = float("nan")
+        x[3, 64:80] = -float("nan")
+    elif case == "inf":
+        x[1, 7] = -float("inf")
+    ld = K + 16 if case == "strided" else K
+    buf = torch.full((rows, ld), float("nan"), dtype=dt)
+    buf[:, :K] = x
+    xg = buf.to(gpu)
+    rd = (lambda t: t.to(dt).float())
+
+    def codes(v):          # e4m3 of fp32 v with the sign kept on NaN, as f32_to_e4m3fn
+        q = v.to(torch.float8_e4m3fn).view(torch.uint8)
+        bad = v.isnan() | (v.abs() > 464)
+        sign = (v.view(torch.int32) >> 31 & 1).to(torch.uint8) * 128
+        return torch.where(bad, sign | 0x7f, q)
+
+    xf = x.float()
+    finite_max = lambda t: torch.where(t.isnan(), torch.zeros_like(t), t).abs()
+    for per_row in (True, False):
+        q = torch.empty(rows, K, device=gpu, dtype=torch.uint8)
+        s = torch.empty(rows, device=gpu, dtype=torch.float32)
+        if per_row:
+            call("omni_fp8_quant_rows_bf16" if bf16 else "omni_fp8_quant_rows", ptr(xg), ld, ptr(q),
+                 ptr(s), rows, K, 0.0, stream())
+            es = finite_max(xf).amax(1) / 448.0
+            v = xf / es[:, None]
+        else:
+            work = torch.empty(lib().omni_fp8_quant_tensor_work(rows), device=gpu,
+                               dtype=torch.float32)
+            call("omni_fp8_quant_tensor", ptr(xg), ld, ptr(q), ptr(s), ptr(work), rows, K,
+                 int(bf16), stream())
+            es = rd(finite_max(xf).max() / 448.0).expand(rows)
+            v = rd(xf / es[:, None])
+        torch.cuda.synchronize()
+        assert torch.equal(s.cpu(), es), (per_row, s, es)
+        got, want = q.cpu(), codes(v.contiguous())
+        free = v.isnan()
+        assert torch.equal(torch.where(free, got & 0x7f, got), torch.where(free, want & 0x7f, want)), per_row
+
+
+@pytest.mark.parametrize("rows,n,bf16", [(1, 128, False), (3, 8960, True), (700, 384, True),
+                                         (64, 8960, False)])
+def test_silu_mul_amax(gpu, rows, n, bf16):
+    """silu_mul_amax: silu_mul's output bit for bit and partial maxima whose maximum is the
+    output's; the per-tensor quantisation from them equals the two-launch one bit for bit."""
+    from omniserver_amd import fused_ops as F
+    from omniserver_amd.linear import FP8Linear
+    say(f"silu_mul_amax rows={rows} n={n} bf16={bf16}")
+    gu = f16((rows, 2 * n), 161).to(torch.bfloat16 if bf16 else torch.float16).to(gpu)
+    want = F.silu_mul(gu)
+    out, parts = F.silu_mul_amax(gu)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert parts.max().item() == out.float().abs().max().item()
+    lin = FP8Linear(f16((128, n), 162, 0.02).to(gpu))
+    a, b = lin.quantize_input(out), lin.quantize_input(out, parts)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    assert torch.equal(lin(out), lin(out, parts))
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 1536, 1024), (8192, 1536, 1152), (8192, 2048, 1024)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_fp8_gemm_forms_agree(gpu, M, N, K, bias):
+    """The three output forms on every tile kernel against one another: the shapes take the
+    256 x 128, 256 x 192 and 256 x 256 tiles; fp16(v) and bf16(v) of the same product differ
+    by their own roundings only, and the first M - 1 rows (the 256 x 128 kernel) are bit-equal
+    to the whole call's."""
+    from omniserver_amd.linear import FP8Linear
+    say(f"fp8 gemm forms M={M} N={N} K={K} bias={bias}")
+    b = f16((N,), 163, 0.5).to(gpu) if bias else None
+    lin = FP8Linear(f16((N, K), 164, 0.02).to(gpu), b, rowwise=True)
+    xq, sa = lin.quantize_input(f16((M, K), 165).to(gpu))
+    outs = {}
+    for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16, lin.OUT_F16):
+        dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
+        y = lin.gemm_out(xq, sa, torch.empty(M, N, device=gpu, dtype=dt), mode)
+        part = lin.gemm_out(xq[:M - 1], sa, torch.empty(M - 1, N, device=gpu, dtype=dt), mode)
+        assert torch.equal(y[:M - 1], part), mode
+        outs[mode] = y.float()
+    ref16 = outs[lin.OUT_F16]
+    # |v| <= |y| + |b|: the bf16 form rounds v, b and their sum (bf16 keeps 8 bits: 2^-8 of
+    # each, together 2^-8 (2 |y| + 2 |b|)), the fp16 form v and the sum (2^-11 of each)
+    tol = (2.0 + 2.0 ** -1) * 2.0 ** -8 * (ref16.abs() + (b.float().abs() if bias else 0.0)) + 1e-6
+    for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16):
+        assert ((outs[mode] - ref16).abs() <= tol).all(), mode
+
+
 def fp8_abs_product(xq, sa, wq, sw):
     """|xq| . |wq|^T * sa * sw: the scale of the terms each output sums."""
     return (xq.float().abs() @ wq.float().abs().t()) * sa.view(-1, 1) * sw.view(1, -1)
