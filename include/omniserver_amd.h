@@ -234,7 +234,7 @@ int omni_prefill_attention_rows(const void* q, int q_stride, const void* k_cache
  * fp16((q - 8) * s), bias added after the fp16 rounding when bias_after_round.  x fp16
  * [M, K] (row stride ldx); weights from omni_gptq_repack.  M <= 64 runs the skinny
  * weight-streaming kernel: ksplit > 1 only with OMNI_EPI_PARTIAL (slices =
- * omni_gemm_slices(K, ksplit)), preset selects the workgroup shape (0..3; SiLU 0..9).
+ * omni_gemm_slices(K, ksplit)), preset selects the workgroup shape (0..3, STORE 0..4; SiLU 0..9).
  * M > 64 (prefill) runs an MFMA GEMM (omni_packed_gemm_pipe's pipeline where its shape and
  * alignment rules hold, else a tiled kernel): OMNI_EPI_STORE / OMNI_EPI_SILU, preset ignored;
  * with OMNI_EPI_STORE, ksplit > 1 splits K over omni_gemm_slices(K, ksplit) slices whose
@@ -287,6 +287,12 @@ int omni_f16_gemm_addnorm(const float* partials, int nparts, const void* residua
 
 /* Number of K slices (whole 128-groups) a split of ksplit gives for K. */
 int omni_gemm_slices(int K, int ksplit);
+
+/* The finish of a split: out fp16 [M][N] (row stride ldo, % 4 == 0) = the OMNI_EPI_STORE
+ * epilogue (bias as in omni_w4a16_gemm) of the sum of nparts fp32 slices [nparts][M][N]
+ * (OMNI_EPI_PARTIAL output, 16-byte aligned) in slice order. */
+int omni_gemm_finish(const float* partial, int nparts, const void* bias, int bias_after_round,
+                     void* out, int ldo, int M, int N, void* stream);
 
 /* load_gptq_llm / gptq_marlin_repack (kernels/marlin_linear.py:94-95, 114-143): AutoGPTQ
  * qweight int32 [K/8, N] + scales fp16 [K/128, N] -> this library's packed int4 layout

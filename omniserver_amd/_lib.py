@@ -84,6 +84,7 @@ SIGNATURES = {
     "omni_vit_attention": [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _F, _P],
     "omni_vit_attention_rows": [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _F, _I, _P],
     "omni_gemm_slices": [_I, _I],
+    "omni_gemm_finish": [_P, _I, _P, _I, _P, _I, _I, _I, _P],
     "omni_lmhead_argmax_grid": [_I],
     "omni_lmhead_max_rows": [_I],
     "omni_lmhead_candidates": [_P, _I, _P, _I, _I, _I, _P, _P, _P, _P],

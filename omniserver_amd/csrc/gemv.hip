@@ -656,6 +656,10 @@ static int dispatch_preset(const GemvArgs& a, int preset, hipStream_t st) {
       case 1: return dispatch_mb<WF, EPI, 1, 8, 1, PF, XS>(a, st);
       case 2: return dispatch_mb<WF, EPI, 1, 4, 4, PF, XS>(a, st);
       case 3: return dispatch_mb<WF, EPI, 2, 4, 2, PF, XS>(a, st);
+      // 16 columns per workgroup, K over its 8 waves: the finished form of few columns
+      case 4:
+        if constexpr (EPI == EPI_STORE) return dispatch_mb<WF, EPI, 1, 1, 8, PF, XS>(a, st);
+        else return OMNI_EINVAL;
       default: return OMNI_EINVAL;
     }
   }
@@ -862,6 +866,59 @@ static int launch_gemm_tile_split(const GemvArgs& a, hipStream_t st) {
   if (rc != OMNI_OK) return rc;
   const int64_t nthr = (int64_t)a.M * (a.N / 4);
   hipLaunchKernelGGL(tile_finish_kernel, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, st, a);
+  OMNI_CHECK_LAUNCH();
+  return OMNI_OK;
+}
+
+// The same sum for a few rows: one wave per workgroup, so that the few outputs spread over the
+// CUs, and up to 16 slices requested at once (a serial loop is a memory round trip a slice).
+__global__ __launch_bounds__(64) void skinny_finish_kernel(GemvArgs a) {
+#pragma clang fp contract(off)
+  const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  const int nq = a.N >> 2;
+  if (i >= (int64_t)a.M * nq) return;
+  const int m = (int)(i / nq), n = (int)(i - (int64_t)m * nq) * 4;
+  const float* p0 = a.partial + (int64_t)m * a.N + n;
+  const int64_t st = (int64_t)a.M * a.N;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < a.KS; b += 16) {
+    f32x4 p[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) p[u] = *(const f32x4*)(p0 + (int64_t)min(b + u, a.KS - 1) * st);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      if (b + u >= a.KS) break;
+      v = b + u == 0 ? p[u] : (f32x4){v[0] + p[u][0], v[1] + p[u][1], v[2] + p[u][2], v[3] + p[u][3]};
+    }
+  }
+  half4_t o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) o[q] = finish_store(v[q], a, n + q);
+  *(half4_t*)(a.out + (int64_t)m * a.ldo + n) = o;
+}
+
+// The finish launch alone: out [M][N] (rows ldo apart) = the EPI_STORE epilogue of the sum of
+// nparts fp32 slices [nparts][M][N] in slice order (omni_*_gemm's EPI_PARTIAL output).
+extern "C" int omni_gemm_finish(const float* partial, int nparts, const void* bias,
+                                int bias_after_round, void* out, int ldo, int M, int N,
+                                void* stream) {
+  if (M < 0 || N <= 0 || nparts < 1) return OMNI_EINVAL;
+  if (N & 3) return OMNI_EUNSUPPORTED;
+  if (M == 0) return OMNI_OK;
+  if (!partial || !out || ldo < N || (ldo & 3)) return OMNI_EINVAL;
+  if (((uintptr_t)partial & 15) || ((uintptr_t)out & 7)) return OMNI_EINVAL;
+  GemvArgs a = {};
+  a.partial = (float*)partial;
+  a.bias = (const half_t*)bias;
+  a.bias_after_round = bias_after_round;
+  a.out = (half_t*)out;
+  a.ldo = ldo;
+  a.M = M;
+  a.N = N;
+  a.KS = nparts;
+  const int64_t grid = ((int64_t)M * (N / 4) + 63) / 64;
+  if (grid > 0x7fffffff) return OMNI_EUNSUPPORTED;
+  hipLaunchKernelGGL(skinny_finish_kernel, dim3((unsigned)grid), dim3(64), 0, (hipStream_t)stream, a);
   OMNI_CHECK_LAUNCH();
   return OMNI_OK;
 }

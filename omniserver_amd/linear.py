@@ -140,6 +140,35 @@ class _Skinny(nn.Module):
             return max(1, min(KG // 2, 256 // tiles))
         return max(1, min(8, KG // 4, 256 // tiles))
 
+    # K slices per 128-group of the finished skinny form where it splits, and the fewest
+    SKINNY_SLICES, SKINNY_MIN_SLICES = (2, 7), 6
+
+    def skinny_plan(self, M: int) -> Tuple[int, int]:
+        """(K slices, preset) of the finished form at up to MAX_SKINNY_M rows; 1 slice: one
+        launch of the store kernel.  Its preset 2 gives a workgroup 64 columns, which at
+        N = 1536 makes 24 of them, and stages all of K's x in LDS, past whose size it crawls.
+        Preset 4 gives 16 columns, K over the 8 waves: while those fit one round of 256
+        workgroups it wins until each has much x to read (rows x K); beyond that fp32 slices
+        over the grid and a finish launch.  MI355X, graph-timed, us (preset 2 / 4 / split):
+        int4 1536 -> 1536 M = 1 5.6 / 4.1 / 6.6, 32 6.8 / 5.8 / 8.0, 64 25.8 / 9.7 / 9.2;
+        8960 -> 1536 M = 1 23.9 / 10.1 / 10.2, 16 38 / 13.2 / 11.3, 32 68 / 20.9 / 12.3, 64 132 /
+        - / 15.8; 3584 -> 3584 M = 32 29.8 / 10.4 / 10.7, 48 42.1 / 13.8 / 12.3; 3584 -> 4608
+        M = 1 9.4 / 10.0 / 9.0, 32 29.6 / 17.1 / 11.3; 1536 -> 8960 M = 48 10.1 / 19.4 / 13.6;
+        fp16 1536 -> 1536 M = 1 7.6 / 4.6 / 7.5, 32 9.2 / 6.8 / 8.7; 8960 -> 1536 M = 1 36.7 /
+        15.7 / 13.6, 32 81 / 25.3 / 15.8, 64 144 / - / 18.6.  Slices: 7 groups each (int4), 3.5
+        (fp16, four times the bytes), from the same sweeps."""
+        KG, blocks = self.K // 128, -(-M // 16)
+        if self.fuse_silu or KG < 4:
+            return 1, self.store_preset
+        if self.N // 16 <= 256:
+            if blocks * KG <= 72:
+                return 1, 4
+        elif blocks * 16 * (self.K + 8) * 2 <= 160 * 1024 or self.N // 64 >= 256:
+            return 1, self.store_preset
+        num, den = self.SKINNY_SLICES
+        ks = min(KG, max(self.SKINNY_MIN_SLICES, KG * num // den))
+        return ks, 3 if KG >= 24 and self.N % 32 == 0 else 1
+
     def forward_out(self, x2d: torch.Tensor, out: torch.Tensor, preset: int | None = None,
                     ksplit: int | None = None):
         """fp16 output (SiLU-fused for gate_up) into out; any number of rows (more than
@@ -147,6 +176,17 @@ class _Skinny(nn.Module):
         along K as tile_ksplit says unless ``ksplit`` is given)."""
         epi = EPI_SILU if self.fuse_silu else EPI_STORE
         M = x2d.shape[0]
+        if 0 < M <= MAX_SKINNY_M and preset is None and ksplit is None:
+            ks, pr = self.skinny_plan(M)
+            if ks == 1:
+                preset = pr
+            elif not ((out.data_ptr() & 7) or (out.stride(0) & 3)):
+                ws = torch.empty(self.partial_slices(ks) * M * self.N, device=x2d.device,
+                                 dtype=torch.float32)
+                S = self.forward_partial(x2d, ws, ks, pr)
+                call("omni_gemm_finish", ptr(ws), S, ptr(self.bias), int(self.fmt == "int4"),
+                     ptr(out), out.stride(0), M, self.N, stream())
+                return out
         ks = self.tile_ksplit(M) if ksplit is None else ksplit
         if M > MAX_SKINNY_M and epi == EPI_STORE and ks > 1:
             ws = torch.empty(self.partial_slices(ks) * M * self.N, device=x2d.device,
@@ -297,6 +337,7 @@ class GPTQLinear(_Skinny):
     """W4A16 GPTQ linear: y = fp16(x . dequant(W)) (+ bias, added after rounding)."""
 
     fmt = "int4"
+    SKINNY_SLICES = (1, 7)
 
     def __init__(self, qweight: torch.Tensor, scales: torch.Tensor, bias=None,
                  group_size: int = 128, fuse_silu: bool = False):

@@ -411,6 +411,38 @@ def test_w4a16_gemm(gpu, M, K, N, bias, silu):
 
 
 @pytest.mark.parametrize("fmt", ["int4", "fp16"])
+@pytest.mark.parametrize("M,K,N,bias", [(1, 8960, 1536, False), (33, 8960, 1536, True),
+                                        (16, 8960, 1536, True), (64, 1536, 2048, True),
+                                        (49, 1536, 272, True), (64, 3584, 272, True),
+                                        (17, 3200, 80, True), (64, 640, 128, False),
+                                        (64, 1536, 4608, True), (3, 512, 16, True)])
+def test_skinny_finished_split(gpu, fmt, M, K, N, bias):
+    """The finished linear at up to 64 rows on each of its forms (16 columns a workgroup, K
+    slices and a finish launch, 64 columns) and at the edges of their rule: within the other linears' tolerance of the fp32 oracle, bias
+    rounded as the format's store epilogue rounds it, nothing written past the output's
+    columns; an output the finish cannot store to (rows 2 halfs apart from 8 bytes) takes the
+    store kernel."""
+    from omniserver_amd.linear import F16Linear, GPTQLinear
+    say(f"skinny finished split {fmt} M={M} K={K} N={N} bias={bias}")
+    b = f16((N,), 75, 0.5) if bias else None
+    if fmt == "int4":
+        qw, sc = _gptq(K, N, 76 + K + N)
+        lin, W = GPTQLinear(qw.to(gpu), sc.to(gpu), None if b is None else b.to(gpu)), ref.gptq_dequant(qw, sc)
+    else:
+        w = f16((N, K), 77, 0.02)
+        lin, W = F16Linear(w.to(gpu), None if b is None else b.to(gpu)), w.float().t()
+    x = f16((M, K), 78)
+    e = ref.linear(x.float(), W, None if b is None else b.float(), bias_after_round=fmt == "int4")
+    tol = 2e-3 * max(1.0, e.abs().max().item())
+    for pad in (8, 2):
+        buf = torch.full((M, N + pad), 7.0, device=gpu, dtype=torch.float16)
+        lin.forward_out(x.to(gpu), buf[:, :N])
+        got = buf.cpu()
+        assert (got[:, :N].float() - e).abs().max().item() <= tol
+        assert (got[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("fmt", ["int4", "fp16"])
 @pytest.mark.parametrize("M", [65, 300])
 @pytest.mark.parametrize("K,N,bias,silu", [
     (1536, 2048, True, False), (8960, 1536, False, False), (1536, 17920, False, True),
