@@ -471,8 +471,7 @@ int omni_fp8_quant_tensor_parts(const void* x, int ldx, void* q, float* scale, c
  *   0  bf16(v) cast to fp16, + fp16 bias in fp16 (row-wise forward, :115-118, 124-125);
  *   1  bf16(v) + bf16(bias) added in bf16 (forward_prequant, :99-108);
  *   2  fp16(v), + fp16 bias in fp16 (per-tensor forward: out_dtype fp16, :119-125; sa and
- *      sw hold one value each, repeated).  This form runs the 256 x 128 kernel where
- *      omni_fp8_gemm_plan names a 256-row big-tile one (their epilogue has no room for it).
+ *      sw hold one value each, repeated).
  * xq [M, K], wq [N, K] e4m3fn; out [M, ldo]; N % 128 == 0, K % 128 == 0; xq, wq and bias
  * 16-byte aligned, sa / sw 4-byte, out 8-byte (else -1). */
 int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, const float* sw,
@@ -494,8 +493,10 @@ int omni_bf16_rne_check(unsigned long long* mismatches, void* stream);
  * persistent 256 x 192 tiles (2 and 3: K >= 1024, M a multiple of 256, N of the width,
  * where rounds of the grid times the tile's work come out below the 256 x 128 tiles', a big
  * tile counted at 0.85 of its size: e.g. every config-4 shape at M = 8192, not N = 1536 at
- * M = 4096); *grid (may be NULL) = its workgroups.  Returns -1 for a shape omni_fp8_gemm
- * rejects. */
+ * M = 4096); 4 the few-row kernel (K >= 512, no big tile, its
+ * estimated time below the 256 x 128 tiles': at K = 8960, N = 1536 to about 1000 rows, at
+ * K = 1536, N = 17920 to 64); *grid (may be NULL) = its workgroups.  Returns -1 for a shape
+ * omni_fp8_gemm rejects. */
 int omni_fp8_gemm_plan(int M, int N, int K, int* grid);
 
 /* ---------------------------------------------------------------- lm_head + greedy */

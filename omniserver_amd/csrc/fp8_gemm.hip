@@ -831,6 +831,103 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
   wait_vmcnt<0>();                             // drain the clamped tail loads before exit
 }
 
+// The same product for few rows (decode batches, short prompts), where a 256 x 128 tile's
+// workgroups are too few and mostly padding: 8960 -> 1536 took 70 us on 12 of them at any
+// M <= 256.  A workgroup owns 16 CT columns x 16 MT rows and its NW waves share K: wave w takes
+// the 128-k steps w, w + NW, .., reading both operands' fragments straight from global memory
+// (a fragment is 16 rows x 128 bytes, whole cache lines), PF steps in flight, and the waves'
+// sums meet in LDS.  Bound by the weight stream at few rows and by the x reads from the L2 as
+// the rows grow (every 16 CT columns read all of a row block's x).
+template <int MT, int CT, int NW, int PF>
+__global__ __launch_bounds__(64 * NW, 1) void fp8_gemm_skinny_kernel(Fp8GemmArgs a) {
+#pragma clang fp contract(off)
+  __shared__ __attribute__((aligned(16))) f32x4 red[NW][CT * MT][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int tiles_n = a.N / (16 * CT);
+  const int L = xcd_logical_block(blockIdx.x, gridDim.x);
+  const int tm = L / tiles_n, tn = L - tm * tiles_n;      // one row block's columns together
+  const int m0 = tm * 16 * MT, n0 = tn * 16 * CT;
+  const int nk = a.K / F8_BK;
+
+  const uint8_t* wp[CT];
+  const uint8_t* xp[MT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) wp[c] = a.wq + (int64_t)(n0 + 16 * c + l16) * a.K + 32 * g4;
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+    xp[t] = a.xq + (int64_t)min(m0 + 16 * t + l16, a.M - 1) * a.K + 32 * g4;
+  struct Frags {
+    i32x8 w[CT], x[MT];
+  };
+  auto load = [&](int ks, Frags& f) {
+    const int64_t k0 = (int64_t)min(ks, nk - 1) * F8_BK;  // past the end: not used
+#pragma unroll
+    for (int c = 0; c < CT; ++c) f.w[c] = *(const i32x8*)(wp[c] + k0);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) f.x[t] = *(const i32x8*)(xp[t] + k0);
+  };
+  f32x4 acc[CT][MT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[c][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  Frags f[PF];
+#pragma unroll
+  for (int u = 0; u < PF; ++u) load(wave + NW * u, f[u]);
+  for (int ks = wave; ks < nk; ks += NW * PF) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      if (ks + NW * u < nk) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+            acc[c][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                f[u].w[c], f[u].x[t], acc[c][t], 0, 0, 0, 127, 0, 127);
+      }
+      load(ks + NW * (u + PF), f[u]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) red[wave][c * MT + t][lane] = acc[c][t];
+  __syncthreads();
+  // lane: columns n0 + 16 c + 4 g4 .. + 3 of row m0 + 16 t + l16; the waves share the tiles
+  for (int i = wave; i < CT * MT; i += NW) {
+    const int c = i / MT, t = i - c * MT;
+    f32x4 v = red[0][i][lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+      const f32x4 p = red[w][i][lane];
+      v = (f32x4){v[0] + p[0], v[1] + p[1], v[2] + p[2], v[3] + p[3]};
+    }
+    const int m = m0 + 16 * t + l16, n = n0 + 16 * c + 4 * g4;
+    if (m >= a.M) continue;
+    const float sm = a.sa[m];
+    const float4 s4 = *(const float4*)(a.sw + n);
+    half4_t bb = (half4_t){0, 0, 0, 0};
+    if (a.bias) bb = *(const half4_t*)(a.bias + n);
+    const bool hb = a.bias != nullptr;
+    const float q0 = (v[0] * sm) * s4.x, q1 = (v[1] * sm) * s4.y, q2 = (v[2] * sm) * s4.z,
+                q3 = (v[3] * sm) * s4.w;
+    uint2 pk;
+    if (a.out_mode == FP8_OUT_BF16) {
+      pk.x = fp8_out_bits2<FP8_OUT_BF16>(q0, q1, bb[0], bb[1], hb);
+      pk.y = fp8_out_bits2<FP8_OUT_BF16>(q2, q3, bb[2], bb[3], hb);
+    } else if (a.out_mode == FP8_OUT_F16) {
+      pk.x = fp8_out_bits2<FP8_OUT_F16>(q0, q1, bb[0], bb[1], hb);
+      pk.y = fp8_out_bits2<FP8_OUT_F16>(q2, q3, bb[2], bb[3], hb);
+    } else {
+      pk.x = fp8_out_bits2<FP8_OUT_F16_VIA_BF16>(q0, q1, bb[0], bb[1], hb);
+      pk.y = fp8_out_bits2<FP8_OUT_F16_VIA_BF16>(q2, q3, bb[2], bb[3], hb);
+    }
+    *(uint2*)((uint16_t*)a.out + (int64_t)m * a.ldo + n) = pk;
+  }
+}
+
 static int num_cus() {
   static int n = 0;
   if (n <= 0) {
@@ -1099,8 +1196,45 @@ static int64_t fp8_big_items(int M, int N, int bc) {
   return (int64_t)(M / F8B_T) * (nb / 256 + (N - nb) / 192);
 }
 
+// The few-row kernel's forms (16 MT rows x 16 CT columns a workgroup) and the one to run, or
+// -1 where the pipelined tiles are estimated ahead.  The estimate, in us, was fitted on one
+// sweep (M 1 .. 1024 at the 2B layer's four shapes) and picks within 1.5 us of its best form:
+// a round of the CUs costs what a workgroup reads, 16 CT weight rows and its share of x, at 35
+// bytes / ns (29 for the 16-wave form, whose waves have the least in flight), and the pipelined
+// kernel's round 0.96 us per 128-k step whatever its tiles hold.  MI355X, us, 256 x 128 tiles /
+// this: 8960 -> 1536 M = 1 71.6 / 8.6, 64 71.5 / 15.7, 128 71.7 / 20.2, 300 73.1 / 26.6, 1024
+// 73.9 / 66.7; 1536 -> 17920 M = 1 17.9 / 10.6, 32 17.8 / 12.9, 64 18.0 / 15.6, 100 18.2 / 23;
+// 1536 -> 2048 M = 1 17.2 / 3.9, 64 17.6 / 6.4, 256 19.3 / 7.3, 1024 19.4 / 15.7.
+struct Fp8Skinny {
+  int mt, ct;
+  double us_per_kb;
+};
+static const Fp8Skinny kFp8Skinny[5] = {
+    {1, 1, 0.034}, {1, 2, 0.0285}, {2, 2, 0.0285}, {4, 2, 0.0285}, {4, 4, 0.0285}};
+
+static int fp8_skinny_form(int M, int N, int K) {
+  if (K / F8_BK < 4) return -1;
+  const int64_t cus = num_cus();
+  auto rounds = [&](int64_t w) { return (double)((w + cus - 1) / cus); };
+  double best = 4.5 + rounds((int64_t)ceil_div(M, 256) * (N / F8_BT)) * (K / F8_BK) * 0.96;
+  int form = -1;
+  for (int i = 0; i < 5; ++i) {
+    const Fp8Skinny& f = kFp8Skinny[i];
+    const int64_t w = (int64_t)ceil_div(M, 16 * f.mt) * (N / (16 * f.ct));
+    const double kb = (16.0 * f.ct + (M < 16 * f.mt ? M : 16 * f.mt)) * K / 1000.0;
+    const double c = 3.0 + rounds(w) * (kb * f.us_per_kb + 0.5);
+    if (c < best) best = c, form = i;
+  }
+  return form;
+}
+
+static int64_t fp8_skinny_grid(int M, int N, int form) {
+  return (int64_t)ceil_div(M, 16 * kFp8Skinny[form].mt) * (N / (16 * kFp8Skinny[form].ct));
+}
+
 // Which kernel omni_fp8_gemm runs for a shape: 0 one tile per workgroup, 1 the pipelined
-// 256 x 128 tiles, 2 the 256 x 256 tiles, 3 the 256 x 192 tiles; and the grid it launches.
+// 256 x 128 tiles, 2 the 256 x 256 tiles, 3 the 256 x 192 tiles, 4 the few-row kernel; and the
+// grid it launches.
 extern "C" int omni_fp8_gemm_plan(int M, int N, int K, int* grid) {
   if (M <= 0 || N <= 0 || K <= 0 || (N % F8_BT) || (K % F8_BK)) return OMNI_EINVAL;
   int kind, g;
@@ -1108,6 +1242,8 @@ extern "C" int omni_fp8_gemm_plan(int M, int N, int K, int* grid) {
   if (bc) {
     const int64_t t = fp8_big_items(M, N, bc);
     kind = bc == 256 ? 2 : 3, g = (int)(t < num_cus() ? t : num_cus());
+  } else if (const int form = fp8_skinny_form(M, N, K); form >= 0) {
+    kind = 4, g = (int)fp8_skinny_grid(M, N, form);
   } else if (K / F8_BK >= 4) {
     const int64_t t8 = (int64_t)ceil_div(M, 256) * (N / F8_BT);
     kind = 1, g = (int)(t8 < num_cus() ? t8 : num_cus());
@@ -1158,6 +1294,16 @@ extern "C" int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, co
       hipLaunchKernelGGL((fp8_gemm_bigp_kernel<8>), dim3((unsigned)grid), dim3(512), 0, (hipStream_t)stream, a);
     else
       hipLaunchKernelGGL((fp8_gemm_bigp_kernel<6>), dim3((unsigned)grid), dim3(512), 0, (hipStream_t)stream, a);
+  } else if (const int form = fp8_skinny_form(M, N, K); form >= 0) {   // few rows
+    const dim3 gd((unsigned)fp8_skinny_grid(M, N, form));
+    hipStream_t st = (hipStream_t)stream;
+    switch (form) {
+      case 0: hipLaunchKernelGGL((fp8_gemm_skinny_kernel<1, 1, 16, 2>), gd, dim3(1024), 0, st, a); break;
+      case 1: hipLaunchKernelGGL((fp8_gemm_skinny_kernel<1, 2, 8, 2>), gd, dim3(512), 0, st, a); break;
+      case 2: hipLaunchKernelGGL((fp8_gemm_skinny_kernel<2, 2, 8, 2>), gd, dim3(512), 0, st, a); break;
+      case 3: hipLaunchKernelGGL((fp8_gemm_skinny_kernel<4, 2, 8, 1>), gd, dim3(512), 0, st, a); break;
+      default: hipLaunchKernelGGL((fp8_gemm_skinny_kernel<4, 4, 4, 1>), gd, dim3(256), 0, st, a); break;
+    }
   } else if (K / F8_BK >= 4) {                    // 8 waves, 256 x 128 tiles, 3 stages
     const int64_t t8 = (int64_t)ceil_div(M, 256) * (N / F8_BT);
     const int grid = (int)(t8 < num_cus() ? t8 : num_cus());

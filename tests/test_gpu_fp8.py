@@ -150,3 +150,37 @@ def test_bf16_rounding_exhaustive(gpu):
     call("omni_bf16_rne_check", ptr(mism), stream())
     torch.cuda.synchronize()
     assert mism.tolist() == [0, 0]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 512, 128), (16, 640, 2048), (17, 8960, 1536),
+                                   (64, 8960, 1536), (65, 1536, 2048), (130, 8960, 1536),
+                                   (300, 1536, 1536), (33, 1536, 17920), (1000, 8960, 1536)])
+def test_fp8_few_rows(gpu, M, K, N, bias):
+    """The few-row kernel in each of its forms (row blocks with one row and one row short of
+    full, K steps that do not divide over its waves, more than one round of workgroups) and
+    every output form, against a float64 product of the same codes: the MFMA's reduced
+    intermediate precision (2^-14 of the absolute product) and the output's roundings; the
+    output's padding columns stay untouched."""
+    from omniserver_amd.linear import FP8Linear
+    kind, grid = plan(M, N, K)
+    say(f"fp8 few rows M={M} K={K} N={N} bias={bias} -> kind {kind}, grid {grid}")
+    assert kind == 4
+    b = f16((N,), 410, 0.5).to(gpu) if bias else None
+    lin = FP8Linear(f16((N, K), 411, 0.02).to(gpu), b, rowwise=True)
+    xq, sa = lin.quantize_input(f16((M, K), 412).to(gpu))
+    e4 = lambda t: t.view(torch.float8_e4m3fn).double()
+    sc = sa.double().view(-1, 1) * lin.weight_scale.double().view(1, -1)
+    v = e4(xq) @ e4(lin.weight_fp8).t() * sc
+    mag = e4(xq).abs() @ e4(lin.weight_fp8).abs().t() * sc
+    bb = b.double() if bias else torch.zeros(N, device=gpu, dtype=torch.float64)
+    for mode, eps in ((lin.OUT_F16_VIA_BF16, 2.0 ** -8), (lin.OUT_BF16, 2.0 ** -8),
+                      (lin.OUT_F16, 2.0 ** -11)):
+        dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
+        buf = torch.full((M, N + 4), 5.0, device=gpu, dtype=dt)
+        lin.gemm_out(xq, sa, buf[:, :N], mode)
+        d = (buf[:, :N].double() - (v + bb)).abs()
+        # v, b (bf16 form) and their sum each rounded once, plus v's fp16 rounding
+        tol = mag * 2.0 ** -14 + (eps + 2.0 ** -11) * (2 * v.abs() + 2 * bb.abs()) + 1e-6
+        assert (d <= tol).all(), (mode, (d - tol).max().item())
+        assert (buf[:, N:] == 5.0).all()
