@@ -499,6 +499,16 @@ int omni_bf16_rne_check(unsigned long long* mismatches, void* stream);
  * omni_fp8_gemm rejects. */
 int omni_fp8_gemm_plan(int M, int N, int K, int* grid);
 
+/* FP8Linear.forward_prequant of a gate|up weight [N, K] followed by silu_mul
+ * (model/qwen2_llm.py:127-131) in one launch: out [M, N / 2] = silu(gate) * up of the products
+ * as out_mode stores them (no bias), in the same type; bit-equal to omni_fp8_gemm +
+ * omni_silu_mul(_bf16).  amax_part (may be NULL): omni_fp8_gemm_silu_grid floats, partial maxima
+ * of |out| for omni_fp8_quant_tensor_parts.  -2 where the grid is 0: shapes omni_fp8_gemm does
+ * not run on the 256 x 256 tiles. */
+int omni_fp8_gemm_silu(const void* xq, const float* sa, const void* wq, const float* sw, void* out,
+                       int ldo, float* amax_part, int M, int N, int K, int out_mode, void* stream);
+int omni_fp8_gemm_silu_grid(int M, int N, int K);
+
 /* ---------------------------------------------------------------- lm_head + greedy */
 
 /* Workgroups (= candidate rows per token) of omni_lmhead_candidates for vocab N. */

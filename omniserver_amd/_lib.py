@@ -52,6 +52,8 @@ SIGNATURES = {
     "omni_fp8_quant_tensor_parts": [_P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
     "omni_fp8_gemm": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "omni_fp8_gemm_plan": [_I, _I, _I, ctypes.POINTER(_I)],
+    "omni_fp8_gemm_silu": [_P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "omni_fp8_gemm_silu_grid": [_I, _I, _I],
     "omni_w4a16_gemm_attn": [_P, _I, _I, _I, _P, _P, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I,
                              _P],
     "omni_f16_gemm_attn": [_P, _I, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],

@@ -71,6 +71,7 @@ struct Fp8GemmArgs {
   int out_mode;          // FP8_OUT_*: how the scaled product is stored (+ bias)
   int n_big;             // persistent 256-column tiles: whole tiles below column n_big, 192-column
                          // tiles from there to N; N elsewhere
+  float* part;           // SiLU form: the grid's partial maxima of |out|, or NULL
 };
 
 // Output forms of the scaled product v = acc * sa[m] * sw[n]:
@@ -558,7 +559,50 @@ __device__ __forceinline__ void fp8_bigp_epilogue(const f32x4 (&acc)[NIW][8], ui
   }
 }
 
-template <int NI, bool TAIL = false>
+template <int MODE, typename ReadCol>
+__device__ __forceinline__ void fp8_bigp_silu(const f32x4 (&acc)[4][8], uint16_t* ob, int ldo,
+                                              const float (&sm)[8], ReadCol read_col, float& amax) {
+#pragma clang fp contract(off)
+  constexpr bool BF = MODE == FP8_OUT_BF16;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {               // gate sub-tile 2 p, up sub-tile 2 p + 1
+    f32x4 sg, su;
+    u32x2 nobias;
+    read_col(2 * p, sg, nobias);
+    read_col(2 * p + 1, su, nobias);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      uint32_t o[2];
+#pragma unroll
+      for (int q = 0; q < 4; q += 2) {
+        // the product's own stored form, then silu_mul's fp32 product rounded to the same type
+        const uint32_t g = fp8_out_bits2<MODE>((acc[2 * p][j][q] * sm[j]) * sg[q],
+                                               (acc[2 * p][j][q + 1] * sm[j]) * sg[q + 1], (half_t)0,
+                                               (half_t)0, false);
+        const uint32_t u = fp8_out_bits2<MODE>((acc[2 * p + 1][j][q] * sm[j]) * su[q],
+                                               (acc[2 * p + 1][j][q + 1] * sm[j]) * su[q + 1],
+                                               (half_t)0, (half_t)0, false);
+        float r[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const unsigned short s =
+              st16f<BF>(silu_mul_f32(ld16f<BF>((unsigned short)(g >> (16 * e))),
+                                     ld16f<BF>((unsigned short)(u >> (16 * e)))));
+          r[e] = ld16f<BF>(s);
+          o[q >> 1] = e ? o[q >> 1] | ((uint32_t)s << 16) : (uint32_t)s;
+        }
+        amax = fmaxf(amax, fmaxf(fabsf(r[0]), fabsf(r[1])));
+      }
+      *(uint2*)(ob + (16 * j * ldo + 16 * p)) = make_uint2(o[0], o[1]);
+    }
+  }
+}
+
+// SILU (256 columns, no bias): w is gate|up [N, K] and out [M, N / 2] = silu(gate) * up of the
+// stored roundings.  A tile's 16-row groups of w alternate between the gate and the up half, so
+// a wave's n sub-tiles pair up in one lane's registers; neither the product nor its re-read
+// crosses memory, and the outputs' maxima per workgroup go to a.part.
+template <int NI, bool TAIL = false, bool SILU = false>
 __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
 #pragma clang fp contract(off)
   constexpr int NS = 2;                       // stages (64 KB + 16 NI * 2 KB each)
@@ -569,6 +613,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
   constexpr int OPS = XLD + WLD;              // operand loads every thread issues per stage
   static_assert(NI == 6 || NI == 8, "tile widths 192 and 256");
   static_assert(!TAIL || NI == 8, "192-column tail tiles after 256-column ones");
+  static_assert(!SILU || (NI == 8 && !TAIL), "gate / up groups pair within a wave");
   __shared__ __attribute__((aligned(1024))) uint8_t xl[NS][F8B_T * F8_ROWB];
   __shared__ __attribute__((aligned(1024))) uint8_t wl[NS][BN * F8_ROWB];
   __shared__ __attribute__((aligned(16))) float scl[2][F8B_T + BN];    // [tile parity][sa | sw]
@@ -614,10 +659,18 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
   const bool has_bias = a.bias != nullptr;
   const uint32_t loff = (uint32_t)lrow * (uint32_t)a.K + (uint32_t)lchunk * 16u;
   const uint32_t rstep = 64u * (uint32_t)a.K;
+  // SILU: LDS row r = 64 u + lrow of w is row n0 / 2 + 32 u + 16 (lrow / 32) + lrow % 16 of the
+  // gate half, or of the up half where lrow / 16 is odd
+  const uint32_t woff = SILU ? (((uint32_t)(lrow >> 4) & 1u) * (uint32_t)(a.N >> 1) +
+                                16u * (uint32_t)(lrow >> 5) + (uint32_t)(lrow & 15)) * (uint32_t)a.K +
+                                   (uint32_t)lchunk * 16u
+                             : loff;
+  const uint32_t wrstep = SILU ? 32u * (uint32_t)a.K : rstep;
   auto issue = [&](int m0, int n0, int ks, int st, int tl) {
     const uint8_t* const xs = a.xq + (int64_t)m0 * a.K;
-    const uint8_t* const ws = a.wq + (int64_t)n0 * a.K;
+    const uint8_t* const ws = a.wq + (int64_t)(SILU ? n0 >> 1 : n0) * a.K;
     const uint32_t k0 = loff + (uint32_t)ks * F8_BK;
+    const uint32_t kw = woff + (uint32_t)ks * F8_BK;
 #pragma unroll
     for (int u = 0; u < XLD; ++u)
       __builtin_amdgcn_global_load_lds((const void*)(xs + (k0 + u * rstep)),
@@ -625,7 +678,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
 #pragma unroll
     for (int u = 0; u < WLD; ++u) {
       if (TAIL && tl && u >= 3) break;  // a 192-column tile's 3 row groups of w
-      __builtin_amdgcn_global_load_lds((const void*)(ws + (k0 + u * rstep)),
+      __builtin_amdgcn_global_load_lds((const void*)(ws + (kw + u * wrstep)),
                                        (lds_void*)((lds_u8*)&wl[st][(64 * u + 8 * wave) * F8_ROWB]), 16, 0, 0);
     }
   };
@@ -644,8 +697,10 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
                                        (lds_void*)((lds_u8*)&scl[p][64 * wave]), 4, 0, 0);
     }
     if (wave < bn / 64) {
-      const uint8_t* const swb = (const uint8_t*)(a.sw + n0 + 64 * wave);
-      __builtin_amdgcn_global_load_lds((const void*)(swb + 4u * ln),
+      const uint8_t* const swb = (const uint8_t*)(a.sw + (SILU ? (n0 >> 1) + 32 * wave : n0 + 64 * wave));
+      const uint32_t col = SILU ? ((ln >> 4) & 1u) * (uint32_t)(a.N >> 1) + 16u * (ln >> 5) + (ln & 15u)
+                                : ln;
+      __builtin_amdgcn_global_load_lds((const void*)(swb + 4u * col),
                                        (lds_void*)((lds_u8*)&scl[p][F8B_T + 64 * wave]), 4, 0, 0);
     }
     if (wave == 0 && has_bias) {
@@ -762,6 +817,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
   wait_vmcnt<OPS>();                          // the scales and stage 0 (issued first)
   barrier_only();
   int sidx = 0;
+  float amax = 0.f;                           // SILU: of what this thread stored
   for (int r = 0; r < my_tiles; ++r) {
     f32x4 acc[NIW][8];   // [n sub-tile][m sub-tile]
 #pragma unroll
@@ -816,7 +872,13 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
                            ((ln & 15u) * (uint32_t)a.ldo + 4u * (ln >> 4));
       auto rc = [&](int i, f32x4& sn, u32x2& bw) { read_col(r & 1, cw, i, sn, bw); };
       const int ni = TAIL && tlc ? 3 : NIW;           // n sub-tiles stored
-      if (a.out_mode == FP8_OUT_BF16)
+      if constexpr (SILU) {
+        uint16_t* const os = (uint16_t*)a.out + (int64_t)(m0c + 128 * wm) * a.ldo + (n0c >> 1) +
+                             32 * wn + ((ln & 15u) * (uint32_t)a.ldo + 4u * (ln >> 4));
+        if (a.out_mode == FP8_OUT_BF16) fp8_bigp_silu<FP8_OUT_BF16>(acc, os, a.ldo, sm, rc, amax);
+        else if (a.out_mode == FP8_OUT_F16) fp8_bigp_silu<FP8_OUT_F16>(acc, os, a.ldo, sm, rc, amax);
+        else fp8_bigp_silu<FP8_OUT_F16_VIA_BF16>(acc, os, a.ldo, sm, rc, amax);
+      } else if (a.out_mode == FP8_OUT_BF16)
         fp8_bigp_epilogue<FP8_OUT_BF16, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
       else if (a.out_mode == FP8_OUT_F16)
         fp8_bigp_epilogue<FP8_OUT_F16, NIW>(acc, ob, a.ldo, sm, rc, has_bias, ni);
@@ -829,6 +891,19 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
     tile_at(r + 2, m0n, n0n, tln);
   }
   wait_vmcnt<0>();                             // drain the clamped tail loads before exit
+  if constexpr (SILU) {
+    if (a.part) {
+      __shared__ float red[8];
+      amax = wave_max(amax);
+      if (lane == 0) red[wave] = amax;
+      __syncthreads();
+      if (tid == 0) {
+#pragma unroll
+        for (int w = 1; w < 8; ++w) amax = fmaxf(amax, red[w]);
+        a.part[blockIdx.x] = amax;
+      }
+    }
+  }
 }
 
 // The same product for few rows (decode batches, short prompts), where a 256 x 128 tile's
@@ -1270,7 +1345,7 @@ extern "C" int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, co
     return OMNI_EINVAL;
   const int64_t tiles = (int64_t)ceil_div(M, F8_BT) * (N / F8_BT);
   if (tiles > 0x7fffffff) return OMNI_EUNSUPPORTED;
-  Fp8GemmArgs a;
+  Fp8GemmArgs a = {};
   a.xq = (const uint8_t*)xq;
   a.sa = sa;
   a.wq = (const uint8_t*)wq;
@@ -1312,6 +1387,48 @@ extern "C" int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, co
   } else {
     hipLaunchKernelGGL(fp8_gemm_kernel, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream, a);
   }
+  OMNI_CHECK_LAUNCH();
+  return OMNI_OK;
+}
+
+// Whether the SiLU form of the persistent tiles runs for a gate|up product, and then its grid
+// (the partial maxima it writes): where omni_fp8_gemm itself would take the 256 x 256 tiles.
+// [8192, 1536] x [17920, 1536]: product 272 us + SiLU-mul 88 us -> 290 us together.
+extern "C" int omni_fp8_gemm_silu_grid(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || (N % 256) || (K % F8_BK)) return 0;
+  if (fp8_big_cols(M, N, K) != 256 || (int64_t)N * K > 0x7fffffff) return 0;
+  const int64_t t = (int64_t)(M / F8B_T) * (N / 256);
+  return (int)(t < num_cus() ? t : num_cus());
+}
+
+extern "C" int omni_fp8_gemm_silu(const void* xq, const float* sa, const void* wq, const float* sw,
+                                  void* out, int ldo, float* amax_part, int M, int N, int K,
+                                  int out_mode, void* stream) {
+  if (M < 0 || N <= 0 || K <= 0) return OMNI_EINVAL;
+  if (out_mode < FP8_OUT_F16_VIA_BF16 || out_mode > FP8_OUT_F16) return OMNI_EINVAL;
+  if (M == 0) return OMNI_OK;
+  const int grid = omni_fp8_gemm_silu_grid(M, N, K);
+  if (!grid) return OMNI_EUNSUPPORTED;
+  if (ldo < N / 2 || (ldo & 3)) return OMNI_EINVAL;
+  if (!xq || !sa || !wq || !sw || !out) return OMNI_EINVAL;
+  if (((uintptr_t)xq & 15) || ((uintptr_t)wq & 15) || ((uintptr_t)sa & 3) || ((uintptr_t)sw & 3) ||
+      ((uintptr_t)out & 7))
+    return OMNI_EINVAL;
+  Fp8GemmArgs a = {};
+  a.xq = (const uint8_t*)xq;
+  a.sa = sa;
+  a.wq = (const uint8_t*)wq;
+  a.sw = sw;
+  a.out = out;
+  a.ldo = ldo;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.out_mode = out_mode;
+  a.n_big = N;
+  a.part = amax_part;
+  hipLaunchKernelGGL((fp8_gemm_bigp_kernel<8, false, true>), dim3((unsigned)grid), dim3(512), 0,
+                     (hipStream_t)stream, a);
   OMNI_CHECK_LAUNCH();
   return OMNI_OK;
 }

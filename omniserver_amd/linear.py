@@ -645,6 +645,27 @@ class FP8Linear(nn.Module):
              ptr(self.bias), ptr(out), out.stride(0), M, self.N, self.K, int(mode), stream())
         return out
 
+    def forward_prequant_silu(self, xq: torch.Tensor, scale: torch.Tensor):
+        """silu_mul(forward_prequant(xq, scale)) of a gate|up weight in one launch, with partial
+        maxima of its magnitudes (``amax_parts``): (out bf16 [..., N / 2], parts), or None
+        where the fused kernel does not run (few or ragged rows, a bias, per-tensor form)."""
+        if not self.rowwise or self.bias is not None:
+            return None
+        xq2 = xq.reshape(-1, self.K)
+        M = xq2.shape[0]
+        grid = lib().omni_fp8_gemm_silu_grid(M, self.N, self.K)
+        if grid == 0:
+            return None
+        if xq2.dtype == torch.float8_e4m3fn:
+            xq2 = xq2.view(torch.uint8)
+        xq2 = xq2.contiguous()
+        sa = scale.reshape(-1).contiguous().float()
+        out = torch.empty(M, self.N // 2, device=xq.device, dtype=torch.bfloat16)
+        parts = torch.empty(grid, device=xq.device, dtype=torch.float32)
+        call("omni_fp8_gemm_silu", ptr(xq2), ptr(sa), ptr(self.weight_fp8), ptr(self.weight_scale),
+             ptr(out), out.stride(0), ptr(parts), M, self.N, self.K, self.OUT_BF16, stream())
+        return out.reshape(*xq.shape[:-1], self.N // 2), parts
+
     def forward_prequant(self, xq: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
         if not self.rowwise:
             raise ValueError("forward_prequant needs the row-wise form (fp8_linear.py:99-103: "

@@ -97,23 +97,31 @@ class MLP(nn.Module):
         self.down_proj = down_proj
 
     def forward(self, x):
+        down = self.down_proj
+        # a per-tensor FP8 down takes its input's maximum from the launch that makes the input
+        amax = (getattr(down.forward, "__func__", None) is FP8Linear.forward and not down.rowwise)
         if isinstance(x, tuple):
             xq, scale = x
-            gu = self.gate_up_proj.forward_prequant(xq, scale)
+            gate_up = self.gate_up_proj
+            if getattr(gate_up.forward_prequant, "__func__", None) is FP8Linear.forward_prequant:
+                fused = gate_up.forward_prequant_silu(xq, scale)
+                if fused is not None:
+                    return self._down(fused[0], fused[1] if amax else None)
+            gu = gate_up.forward_prequant(xq, scale)
         else:
             gu = self.gate_up_proj(x)
         if getattr(self.gate_up_proj, "fuse_silu", False):
-            out = gu
-        elif (getattr(self.down_proj.forward, "__func__", None) is FP8Linear.forward
-                and not self.down_proj.rowwise and gu.numel()):
-            # a per-tensor FP8 down: its input's maximum comes out of the SiLU-mul's launch
-            out, parts = F.silu_mul_amax(gu)
-            return self.down_proj(out, parts)
-        else:
-            out = F.silu_mul(gu)
-        if out.dtype != torch.float16 and not hasattr(self.down_proj, "forward_prequant"):
-            out = out.to(torch.float16)
-        return self.down_proj(out)
+            return self._down(gu, None)
+        if amax and gu.numel():
+            return self._down(*F.silu_mul_amax(gu))
+        return self._down(F.silu_mul(gu), None)
+
+    def _down(self, act, parts):
+        if parts is not None:
+            return self.down_proj(act, parts)
+        if act.dtype != torch.float16 and not hasattr(self.down_proj, "forward_prequant"):
+            act = act.to(torch.float16)
+        return self.down_proj(act)
 
 
 class DecoderLayer(nn.Module):

@@ -1362,6 +1362,33 @@ def test_fp8_gemm_forms_agree(gpu, M, N, K, bias):
         assert ((outs[mode] - ref16).abs() <= tol).all(), mode
 
 
+@pytest.mark.parametrize("M,N,K", [(8192, 2048, 1024), (2048, 17920, 1536)])
+def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
+    """The gate|up product with the SiLU-mul in its epilogue: every output form bit-equal to
+    the product followed by silu_mul, more and fewer tiles than CUs, the partial maxima's
+    maximum the output's, rows past the output's columns untouched; shapes off the 256 x 256
+    tiles are refused."""
+    from omniserver_amd import fused_ops as F
+    from omniserver_amd._lib import call, lib, ptr, stream
+    from omniserver_amd.linear import FP8Linear
+    say(f"fp8 gemm + silu M={M} N={N} K={K}")
+    lin = FP8Linear(f16((N, K), 166, 0.05).to(gpu), rowwise=True)
+    xq, sa = lin.quantize_input(f16((M, K), 167).to(gpu))
+    grid = lib().omni_fp8_gemm_silu_grid(M, N, K)
+    assert grid > 0 and lib().omni_fp8_gemm_silu_grid(M - 1, N, K) == 0
+    for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16, lin.OUT_F16):
+        dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
+        want = F.silu_mul(lin.gemm_out(xq, sa, torch.empty(M, N, device=gpu, dtype=dt), mode))
+        buf = torch.full((M, N // 2 + 4), 3.0, device=gpu, dtype=dt)
+        parts = torch.empty(grid, device=gpu, dtype=torch.float32)
+        call("omni_fp8_gemm_silu", ptr(xq), ptr(sa), ptr(lin.weight_fp8), ptr(lin.weight_scale),
+             ptr(buf), buf.stride(0), ptr(parts), M, N, K, mode, stream())
+        got = buf[:, :N // 2].contiguous()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), mode
+        assert parts.max().item() == want.float().abs().max().item()
+        assert (buf[:, N // 2:] == 3.0).all()
+
+
 def fp8_abs_product(xq, sa, wq, sw):
     """|xq| . |wq|^T * sa * sw: the scale of the terms each output sums."""
     return (xq.float().abs() @ wq.float().abs().t()) * sa.view(-1, 1) * sw.view(1, -1)
