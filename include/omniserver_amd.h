@@ -490,7 +490,7 @@ int omni_bf16_rne_check(unsigned long long* mismatches, void* stream);
  * 1 the pipelined persistent 256 x 128 tiles, 2 the persistent 256 x 256 tiles (where whole
  * tiles would leave the grid's last round partly idle, the columns past whole rounds as
  * 256 x 192 tiles after them, at most one per CU: config 4's gate_up at M = 8192), 3 the
- * persistent 256 x 192 tiles (2 and 3: K >= 1024, M a multiple of 256, N of the width,
+ * persistent 256 x 192 tiles (2 and 3: K >= 1024, M >= 256, N a multiple of the width,
  * where rounds of the grid times the tile's work come out below the 256 x 128 tiles', a big
  * tile counted at 0.85 of its size: e.g. every config-4 shape at M = 8192, not N = 1536 at
  * M = 4096); 4 the few-row kernel (K >= 512, no big tile, its
@@ -503,8 +503,8 @@ int omni_fp8_gemm_plan(int M, int N, int K, int* grid);
  * (model/qwen2_llm.py:127-131) in one launch: out [M, N / 2] = silu(gate) * up of the products
  * as out_mode stores them (no bias), in the same type; bit-equal to omni_fp8_gemm +
  * omni_silu_mul(_bf16).  amax_part (may be NULL): omni_fp8_gemm_silu_grid floats, partial maxima
- * of |out| for omni_fp8_quant_tensor_parts.  -2 where the grid is 0: shapes omni_fp8_gemm does
- * not run on the 256 x 256 tiles. */
+ * of |out| for omni_fp8_quant_tensor_parts.  -2 where the grid is 0: M < 256,
+ * K < 1024, N not a multiple of 256, or shapes the two launches are faster for. */
 int omni_fp8_gemm_silu(const void* xq, const float* sa, const void* wq, const float* sw, void* out,
                        int ldo, float* amax_part, int M, int N, int K, int out_mode, void* stream);
 int omni_fp8_gemm_silu_grid(int M, int N, int K);

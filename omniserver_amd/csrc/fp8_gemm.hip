@@ -532,6 +532,9 @@ __device__ __forceinline__ uint32_t fp8_out_bits2(float v0, float v1, half_t b0,
 // (fp8_tail_cols); such a tile loads 3 of the 4 row groups of w, reads its wave's 3 n
 // sub-tiles from 48 wn plus a fourth fragment from the slot's next 16 rows (unused), and
 // stores 3 of its 4 n sub-tiles, so both kinds share the loop's code and registers.
+// Rows past the last multiple of 256 take a tile that ends at row M - 1 and repeats rows of the
+// tile before it (M >= 256): the same sums in the same order, so the two write the same bytes,
+// and neither the loads nor the stores need a bound.
 template <int MODE, int NIW, typename ReadCol>
 __device__ __forceinline__ void fp8_bigp_epilogue(const f32x4 (&acc)[NIW][8], uint16_t* ob, int ldo,
                                                   const float (&sm)[8], ReadCol read_col,
@@ -627,7 +630,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
   const int g4 = lane >> 4;
 
   const int tiles_n = a.n_big / BN;
-  const int tiles_m = a.M / F8B_T;
+  const int tiles_m = (a.M + F8B_T - 1) / F8B_T;
   const int tiles = tiles_m * tiles_n;
   // 256-column tiles: the columns past n_big as 256 x 192 tiles after every whole tile (a
   // grid whose whole tiles fill R rounds exactly then ends with at most one such tile per CU)
@@ -649,7 +652,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_bigp_kernel(Fp8GemmArgs a) {
       n0 = a.n_big + tn * 192;
       tl = 1;
     }
-    m0 = tm * F8B_T;
+    m0 = min(tm * F8B_T, a.M - F8B_T);     // the last tile ends at row M - 1
   };
 
   const int lrow = 8 * wave + (lane >> 3);
@@ -1237,7 +1240,7 @@ extern "C" int omni_fp8_quant_tensor(const void* x, int ldx, void* q, float* sca
 // split exists.
 static int fp8_tail_cols(int M, int N) {
   const int64_t cus = num_cus();
-  const int64_t tm = M / F8B_T, tn = N / 256;
+  const int64_t tm = ceil_div(M, F8B_T), tn = N / 256;
   const int64_t tiles = tm * tn;
   const int64_t R = tiles / cus;
   if (R == 0 || tiles % cus == 0 || (R * cus) % tm) return N;
@@ -1247,28 +1250,31 @@ static int fp8_tail_cols(int M, int N) {
   return (int)(nb * 256);
 }
 
-static int fp8_big_cols(int M, int N, int K) {
-  if (K < 1024 || (M % F8B_T)) return 0;
+// *cost: the choice's rounds, in those of the 256 x 128 tiles.
+static int fp8_big_cols(int M, int N, int K, double* cost = nullptr) {
+  if (K < 1024 || M < F8B_T) return 0;
   const int64_t cus = num_cus();
   auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
-  double best = (double)rounds((int64_t)(M / 256) * (N / F8_BT));   // pipelined tiles
+  double best = (double)rounds((int64_t)ceil_div(M, 256) * (N / F8_BT));   // pipelined tiles
   int cols = 0;
   for (int bn : {256, 192}) {
     if (N % bn) continue;
-    const int64_t t = (int64_t)(M / F8B_T) * (N / bn);
-    // with a 192-column tail (fp8_tail_cols) the last round is 0.75 of a whole one
-    const double r = bn == 256 && fp8_tail_cols(M, N) < N ? (double)(t / cus) + 0.75 : (double)rounds(t);
+    const int64_t t = (int64_t)ceil_div(M, F8B_T) * (N / bn);
+    // with a 192-column tail (fp8_tail_cols) the last round is 0.8 of a whole one (K 1536 ->
+    // N 17920, M = 1000: 1 + tail 57.3 us, 3 rounds of 256 x 128 tiles 53.7)
+    const double r = bn == 256 && fp8_tail_cols(M, N) < N ? (double)(t / cus) + 0.8 : (double)rounds(t);
     const double c = r * (bn / 128.0) * 0.85;
     if (c < best) best = c, cols = bn;
   }
+  if (cost) *cost = best;
   return cols;
 }
 
 // Items of the persistent big kernel (whole tiles plus the 192-column tail tiles).
 static int64_t fp8_big_items(int M, int N, int bc) {
-  if (bc != 256) return (int64_t)(M / F8B_T) * (N / bc);
+  if (bc != 256) return (int64_t)ceil_div(M, F8B_T) * (N / bc);
   const int nb = fp8_tail_cols(M, N);
-  return (int64_t)(M / F8B_T) * (nb / 256 + (N - nb) / 192);
+  return (int64_t)ceil_div(M, F8B_T) * (nb / 256 + (N - nb) / 192);
 }
 
 // The few-row kernel's forms (16 MT rows x 16 CT columns a workgroup) and the one to run, or
@@ -1287,7 +1293,7 @@ struct Fp8Skinny {
 static const Fp8Skinny kFp8Skinny[5] = {
     {1, 1, 0.034}, {1, 2, 0.0285}, {2, 2, 0.0285}, {4, 2, 0.0285}, {4, 4, 0.0285}};
 
-static int fp8_skinny_form(int M, int N, int K) {
+static int fp8_skinny_form(int M, int N, int K, double* us = nullptr) {
   if (K / F8_BK < 4) return -1;
   const int64_t cus = num_cus();
   auto rounds = [&](int64_t w) { return (double)((w + cus - 1) / cus); };
@@ -1300,6 +1306,7 @@ static int fp8_skinny_form(int M, int N, int K) {
     const double c = 3.0 + rounds(w) * (kb * f.us_per_kb + 0.5);
     if (c < best) best = c, form = i;
   }
+  if (us) *us = best;
   return form;
 }
 
@@ -1392,13 +1399,23 @@ extern "C" int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, co
 }
 
 // Whether the SiLU form of the persistent tiles runs for a gate|up product, and then its grid
-// (the partial maxima it writes): where omni_fp8_gemm itself would take the 256 x 256 tiles.
-// [8192, 1536] x [17920, 1536]: product 272 us + SiLU-mul 88 us -> 290 us together.
+// (the partial maxima it writes): where its rounds (whole 256 x 256 tiles) cost less than what
+// omni_fp8_gemm would run and the SiLU-mul pass (3 N bytes a row at 5 bytes / ns), at 0.96 us
+// per 128-k step of a 256 x 128 round as above.  K 1536 -> N 17920, us, this / product then
+// SiLU-mul: M = 8192 237 / 378, 5000 158 / 227, 1000 52.6 / 64.7, 300 29.3 / 41.8.
 extern "C" int omni_fp8_gemm_silu_grid(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || (N % 256) || (K % F8_BK)) return 0;
-  if (fp8_big_cols(M, N, K) != 256 || (int64_t)N * K > 0x7fffffff) return 0;
-  const int64_t t = (int64_t)(M / F8B_T) * (N / 256);
-  return (int)(t < num_cus() ? t : num_cus());
+  if (M < F8B_T || N <= 0 || K < 1024 || (N % 256) || (K % F8_BK)) return 0;
+  if ((int64_t)N * K > 0x7fffffff) return 0;
+  const int64_t t = (int64_t)ceil_div(M, F8B_T) * (N / 256);
+  if (t > 0x7fffffff) return 0;
+  const int64_t cus = num_cus();
+  const double step_us = (K / F8_BK) * 0.96;
+  double rounds, two;
+  if (fp8_big_cols(M, N, K, &rounds)) two = 4.5 + rounds * step_us;
+  else fp8_skinny_form(M, N, K, &two);
+  two += (double)M * N * 3.0 / 5e6;
+  if (4.5 + (double)((t + cus - 1) / cus) * 2 * 0.85 * step_us >= two) return 0;
+  return (int)(t < cus ? t : cus);
 }
 
 extern "C" int omni_fp8_gemm_silu(const void* xq, const float* sa, const void* wq, const float* sw,

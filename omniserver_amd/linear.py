@@ -645,26 +645,54 @@ class FP8Linear(nn.Module):
              ptr(self.bias), ptr(out), out.stride(0), M, self.N, self.K, int(mode), stream())
         return out
 
+    def _rows(self, x: torch.Tensor) -> torch.Tensor:
+        x2d = x.reshape(-1, self.K)
+        if not x2d.is_contiguous():
+            x2d = x2d.contiguous()
+        require_cuda(x2d)
+        if x2d.dtype not in (torch.float16, torch.bfloat16):
+            raise TypeError(f"expected fp16 or bf16 activations, got {x2d.dtype}")
+        return x2d
+
+    def _silu_out(self, xq2: torch.Tensor, sa: torch.Tensor, grid: int, mode: int):
+        M = xq2.shape[0]
+        out = torch.empty(M, self.N // 2, device=xq2.device,
+                          dtype=torch.bfloat16 if mode == self.OUT_BF16 else torch.float16)
+        parts = torch.empty(grid, device=xq2.device, dtype=torch.float32)
+        call("omni_fp8_gemm_silu", ptr(xq2), ptr(sa), ptr(self.weight_fp8), ptr(self.weight_scale),
+             ptr(out), out.stride(0), ptr(parts), M, self.N, self.K, int(mode), stream())
+        return out, parts
+
+    def _silu_grid(self, M: int) -> int:
+        return 0 if self.bias is not None else lib().omni_fp8_gemm_silu_grid(M, self.N, self.K)
+
     def forward_prequant_silu(self, xq: torch.Tensor, scale: torch.Tensor):
         """silu_mul(forward_prequant(xq, scale)) of a gate|up weight in one launch, with partial
         maxima of its magnitudes (``amax_parts``): (out bf16 [..., N / 2], parts), or None
-        where the fused kernel does not run (few or ragged rows, a bias, per-tensor form)."""
-        if not self.rowwise or self.bias is not None:
+        where the fused kernel does not run (few rows, a bias, per-tensor form)."""
+        if not self.rowwise:
             return None
         xq2 = xq.reshape(-1, self.K)
-        M = xq2.shape[0]
-        grid = lib().omni_fp8_gemm_silu_grid(M, self.N, self.K)
+        grid = self._silu_grid(xq2.shape[0])
         if grid == 0:
             return None
         if xq2.dtype == torch.float8_e4m3fn:
             xq2 = xq2.view(torch.uint8)
-        xq2 = xq2.contiguous()
-        sa = scale.reshape(-1).contiguous().float()
-        out = torch.empty(M, self.N // 2, device=xq.device, dtype=torch.bfloat16)
-        parts = torch.empty(grid, device=xq.device, dtype=torch.float32)
-        call("omni_fp8_gemm_silu", ptr(xq2), ptr(sa), ptr(self.weight_fp8), ptr(self.weight_scale),
-             ptr(out), out.stride(0), ptr(parts), M, self.N, self.K, self.OUT_BF16, stream())
+        out, parts = self._silu_out(xq2.contiguous(), scale.reshape(-1).contiguous().float(), grid,
+                                    self.OUT_BF16)
         return out.reshape(*xq.shape[:-1], self.N // 2), parts
+
+    def forward_silu(self, x: torch.Tensor):
+        """silu_mul(forward(x)) with partial maxima of its magnitudes, as
+        forward_prequant_silu: (out fp16 [..., N / 2], parts), or None."""
+        x2d = self._rows(x)
+        grid = self._silu_grid(x2d.shape[0])
+        if grid == 0:
+            return None
+        xq, sa = self.quantize_input(x2d)
+        out, parts = self._silu_out(xq, sa, grid,
+                                    self.OUT_F16_VIA_BF16 if self.rowwise else self.OUT_F16)
+        return out.reshape(*x.shape[:-1], self.N // 2), parts
 
     def forward_prequant(self, xq: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
         if not self.rowwise:
@@ -681,12 +709,7 @@ class FP8Linear(nn.Module):
     def forward(self, x: torch.Tensor, amax_parts: torch.Tensor | None = None) -> torch.Tensor:
         """fp16 or bf16 x (the bf16 silu_mul output of the fused FP8 MLP route,
         qwen2_llm.py:132-134) -> fp16.  ``amax_parts``: see quantize_input."""
-        x2d = x.reshape(-1, self.K)
-        if not x2d.is_contiguous():
-            x2d = x2d.contiguous()
-        require_cuda(x2d)
-        if x2d.dtype not in (torch.float16, torch.bfloat16):
-            raise TypeError(f"expected fp16 or bf16 activations, got {x2d.dtype}")
+        x2d = self._rows(x)
         xq, sa = self.quantize_input(x2d, amax_parts)
         out = torch.empty(x2d.shape[0], self.N, device=x.device, dtype=torch.float16)
         self.gemm_out(xq, sa, out, self.OUT_F16_VIA_BF16 if self.rowwise else self.OUT_F16)

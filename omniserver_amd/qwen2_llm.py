@@ -82,6 +82,12 @@ class Attention(nn.Module):
         self.o_proj = o_proj
 
 
+def _is_method(mod, name: str, cls) -> bool:
+    """Whether mod.name is cls's own, on a module without hooks that would miss it."""
+    return (getattr(getattr(mod, name, None), "__func__", None) is getattr(cls, name)
+            and not (mod._forward_pre_hooks or mod._forward_hooks))
+
+
 class MLP(nn.Module):
     """model/qwen2_llm.py:115-134.  gate_up -> silu_mul -> down, where
     * a gate_up module built with the SiLU epilogue (``fuse_silu``) already emits
@@ -97,19 +103,21 @@ class MLP(nn.Module):
         self.down_proj = down_proj
 
     def forward(self, x):
-        down = self.down_proj
+        down, gate_up = self.down_proj, self.gate_up_proj
         # a per-tensor FP8 down takes its input's maximum from the launch that makes the input
-        amax = (getattr(down.forward, "__func__", None) is FP8Linear.forward and not down.rowwise)
+        amax = _is_method(down, "forward", FP8Linear) and not down.rowwise
+        fused = None
         if isinstance(x, tuple):
             xq, scale = x
-            gate_up = self.gate_up_proj
-            if getattr(gate_up.forward_prequant, "__func__", None) is FP8Linear.forward_prequant:
+            if _is_method(gate_up, "forward_prequant", FP8Linear):
                 fused = gate_up.forward_prequant_silu(xq, scale)
-                if fused is not None:
-                    return self._down(fused[0], fused[1] if amax else None)
-            gu = gate_up.forward_prequant(xq, scale)
+            gu = gate_up.forward_prequant(xq, scale) if fused is None else None
         else:
-            gu = self.gate_up_proj(x)
+            if _is_method(gate_up, "forward", FP8Linear):
+                fused = gate_up.forward_silu(x)
+            gu = gate_up(x) if fused is None else None
+        if fused is not None:
+            return self._down(fused[0], fused[1] if amax else None)
         if getattr(self.gate_up_proj, "fuse_silu", False):
             return self._down(gu, None)
         if amax and gu.numel():

@@ -1340,8 +1340,8 @@ def test_silu_mul_amax(gpu, rows, n, bf16):
 def test_fp8_gemm_forms_agree(gpu, M, N, K, bias):
     """The three output forms on every tile kernel against one another: the shapes take the
     256 x 128, 256 x 192 and 256 x 256 tiles; fp16(v) and bf16(v) of the same product differ
-    by their own roundings only, and the first M - 1 rows (the 256 x 128 kernel) are bit-equal
-    to the whole call's."""
+    by their own roundings only, and the first M - 1 rows (a ragged row count: the 256 x 128
+    tiles or a big tile that ends at the last row) are bit-equal to the whole call's."""
     from omniserver_amd.linear import FP8Linear
     say(f"fp8 gemm forms M={M} N={N} K={K} bias={bias}")
     b = f16((N,), 163, 0.5).to(gpu) if bias else None
@@ -1362,12 +1362,44 @@ def test_fp8_gemm_forms_agree(gpu, M, N, K, bias):
         assert ((outs[mode] - ref16).abs() <= tol).all(), mode
 
 
-@pytest.mark.parametrize("M,N,K", [(8192, 2048, 1024), (2048, 17920, 1536)])
+@pytest.mark.parametrize("M,N,K", [(257, 36864, 1024), (7937, 1536, 1024), (8190, 1536, 1152),
+                                   (8191, 2048, 1024), (2047, 17920, 1536), (8250, 17920, 1024)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_fp8_gemm_big_tiles_ragged_rows(gpu, M, N, K, bias):
+    """Row counts off a multiple of 256 on the big tiles (a last row tile that repeats up to
+    255 rows of the one before it; 256 and 192 columns, with and without 192-column tail tiles):
+    every output form bit-equal to pieces of the rows on the 256 x 128 tiles, the output's
+    padding columns and the rows after it untouched."""
+    import ctypes
+    from omniserver_amd._lib import lib
+    from omniserver_amd.linear import FP8Linear
+    kind = lambda m: lib().omni_fp8_gemm_plan(m, N, K, ctypes.byref(ctypes.c_int()))
+    piece = next(m for m in (3500, 1700, 1000, 500, 250, 200, 128) if kind(m) == 1)
+    say(f"fp8 gemm ragged M={M} N={N} K={K} bias={bias} kind {kind(M)} pieces {piece}")
+    assert kind(M) in (2, 3)
+    b = f16((N,), 168, 0.5).to(gpu) if bias else None
+    lin = FP8Linear(f16((N, K), 169, 0.02).to(gpu), b, rowwise=True)
+    xq, sa = lin.quantize_input(f16((M, K), 170).to(gpu))
+    for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16, lin.OUT_F16):
+        dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
+        buf = torch.full((M + 2, N + 4), 3.0, device=gpu, dtype=dt)
+        lin.gemm_out(xq, sa, buf[:M, :N], mode)
+        assert (buf[M:] == 3.0).all() and (buf[:, N:] == 3.0).all()
+        for o in range(0, M, piece):
+            o = min(o, M - piece)
+            want = lin.gemm_out(xq[o:o + piece], sa[o:o + piece],
+                                torch.empty(piece, N, device=gpu, dtype=dt), mode)
+            assert torch.equal(buf[o:o + piece, :N].contiguous().view(torch.int16),
+                               want.view(torch.int16)), (mode, o)
+
+
+@pytest.mark.parametrize("M,N,K", [(8192, 2048, 1024), (2048, 17920, 1536), (8191, 2048, 1024),
+                                   (1937, 17920, 1536)])
 def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
     """The gate|up product with the SiLU-mul in its epilogue: every output form bit-equal to
-    the product followed by silu_mul, more and fewer tiles than CUs, the partial maxima's
-    maximum the output's, rows past the output's columns untouched; shapes off the 256 x 256
-    tiles are refused."""
+    the product followed by silu_mul, more and fewer tiles than CUs, a last row
+    tile that repeats rows, the partial maxima's maximum the output's, columns past the output untouched; shapes off
+    the 256 x 256 tiles are refused."""
     from omniserver_amd import fused_ops as F
     from omniserver_amd._lib import call, lib, ptr, stream
     from omniserver_amd.linear import FP8Linear
@@ -1375,7 +1407,7 @@ def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
     lin = FP8Linear(f16((N, K), 166, 0.05).to(gpu), rowwise=True)
     xq, sa = lin.quantize_input(f16((M, K), 167).to(gpu))
     grid = lib().omni_fp8_gemm_silu_grid(M, N, K)
-    assert grid > 0 and lib().omni_fp8_gemm_silu_grid(M - 1, N, K) == 0
+    assert grid > 0 and lib().omni_fp8_gemm_silu_grid(255, N, K) == 0
     for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16, lin.OUT_F16):
         dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
         want = F.silu_mul(lin.gemm_out(xq, sa, torch.empty(M, N, device=gpu, dtype=dt), mode))
@@ -1387,6 +1419,28 @@ def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), mode
         assert parts.max().item() == want.float().abs().max().item()
         assert (buf[:, N // 2:] == 3.0).all()
+
+
+@pytest.mark.parametrize("rowwise", [False, True])
+@pytest.mark.parametrize("M", [1, 255, 256, 300, 1000, 1025])
+def test_fp8_mlp_fused_silu(gpu, M, rowwise):
+    """The FP8 MLP on both sides of the fused gate|up rule: bit-equal to its linears called one
+    by one with silu_mul between them, also where a forward hook keeps it off the fused form."""
+    from omniserver_amd import fused_ops as F
+    from omniserver_amd.linear import FP8Linear
+    from omniserver_amd.qwen2_llm import MLP
+    say(f"fp8 mlp fused silu M={M} rowwise={rowwise}")
+    gu = FP8Linear(f16((17920, 1536), 171, 0.05).to(gpu), rowwise=rowwise)
+    down = FP8Linear(f16((1536, 8960), 172, 0.05).to(gpu), rowwise=rowwise)
+    x = f16((M, 1536), 173).to(gpu)
+    mlp = MLP(gu, down)
+    want = down(F.silu_mul(gu(x)))
+    assert torch.equal(mlp(x), want)
+    seen = []
+    gu.register_forward_hook(lambda m, args, out: seen.append(out.shape))
+    down.register_forward_pre_hook(lambda m, args: seen.append(len(args)))
+    assert torch.equal(mlp(x), want)
+    assert seen == [(M, 17920), 1]
 
 
 def fp8_abs_product(xq, sa, wq, sw):
