@@ -531,8 +531,10 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
   gp_wait_vmcnt<0>();                  // drain the clamped tail loads before exit
 }
 
-// Persistent 256 x 256 or 256 x 192 tiles for the packed fp16 weights (STORE without a
-// bias, SILU (256 columns) and PARTIAL epilogues, M a multiple of 256, N of the tile width):
+// Persistent 256 x 256 or 256 x 192 (PARTIAL) tiles for the packed fp16 weights (every
+// epilogue but RESID, M >= 256, N a multiple of the tile width; rows past the last multiple of
+// 256 take a tile that ends at row M - 1 and repeats rows of the tile before it: the same
+// bytes written twice, no bound on loads or stores):
 // 8 waves (two per SIMD: 2 along m x 4 along n), each owning a 128 (m) x 16 NIW (n) block,
 // so every operand byte staged through LDS feeds twice the MFMA work it feeds in the
 // 256 x 128 tiles above; two stages of 32 KB of x and 8 NIW KB of w (x rows XOR-swizzled as
@@ -545,9 +547,12 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
 // leave CUs idle), read and stored by the same code for NIW / 2 column tiles per wave.
 // PARTIAL writes each K slice's fp32 sums to part[slice][M][N] for the consumer to add in
 // slice order (config 5's down projection at M = 4096: 128 tiles of 256 x 192 in two
-// slices fill the 256 CUs once).  (Biased
-// linears, e.g. qkv, stay on the kernel above: with the bias staging beside the
-// accumulators a four-wave form of this kernel spilled.)  Same k order per output as the
+// slices fill the 256 CUs once).  A
+// tile's biases ride with its first stage into an LDS slot of their own (two, by tile parity):
+// read from global memory in the epilogue they would wait for the next tile's stages.  The
+// vision tower's linears, 256 x 128 tiles / this, us: 1280 -> 5120 + QGELU at 3872 rows 76.9 /
+// 75.5, 2100 52.4 / 46.5, 2852 54 / 49.5; 1280 -> 3840 at 3872 49.4 / 47.2, 2852 47.9 / 42.8;
+// 5120 -> 5120 + GELU at 2100 165 / 141.6.  Same k order per output as the
 // kernel above within a slice: one-slice results equal its bit for bit.  MI355X, us
 // (256 x 128 or 128 x 192 / this, interleaved, median of 7): M = 4096 gate_up + SiLU
 // 240.1 / 222.6; M = 8192 gate_up 469.7 / 397.5, down 238.6 / 200.2 (four waves of 128 x 128:
@@ -564,9 +569,9 @@ __device__ __forceinline__ uint32_t gp_lane_now() {
 template <int EPI, int NIW>
 __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
 #pragma clang fp contract(off)
-  static_assert(((EPI == GP_STORE || EPI == GP_PARTIAL) && (NIW == 3 || NIW == 4)) ||
-                    (EPI == GP_SILU && NIW == 4),
-                "STORE / PARTIAL at 192 or 256 columns, SILU at 256");
+  constexpr bool BIAS = EPI == GP_STORE || EPI == GP_QGELU || EPI == GP_GELU;
+  static_assert((EPI == GP_PARTIAL && NIW == 3) || ((EPI == GP_PARTIAL || EPI == GP_SILU || BIAS) && NIW == 4),
+                "PARTIAL at 192 or 256 columns, the others at 256");
   constexpr int NS = 2;
   constexpr int BM = 256;               // tile rows
   constexpr int BN = 64 * NIW;          // tile columns
@@ -575,6 +580,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
   constexpr int NV = 2 * NIW + 16;      // operand fragments per step: w 2 NIW, then x 16
   __shared__ __attribute__((aligned(1024))) uint8_t xl[NS][BM * GP_ROWB];
   __shared__ __attribute__((aligned(1024))) uint8_t wl[NS][BN * GP_ROWB];
+  __shared__ __attribute__((aligned(16))) half_t bsl[2][BIAS ? 512 : 8];   // [tile parity][bias]
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -584,7 +590,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
   const int g4 = lane >> 4;
 
   const int tiles_n = a.n_big / BN;
-  const int tiles_m = a.M / BM;
+  const int tiles_m = (a.M + BM - 1) / BM;
   const int tiles = tiles_m * tiles_n;
   const int items_big = tiles * a.KS;                       // slice-major: item = s tiles + tile
   // the columns past n_big in 256 x (BN / 2) half tiles, after every whole tile: a grid whose
@@ -614,7 +620,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
       t.n0 = a.n_big + tn * (BN / 2);
       t.half = 1;
     }
-    t.m0 = tm * BM;
+    t.m0 = min(tm * BM, a.M - BM);       // the last tile ends at row M - 1
     // slices are whole 128-k groups (pairs of steps), as in the kernel above
     t.kb = 2 * (t.sl * (nk / 2) / a.KS);
     t.kc = 2 * ((t.sl + 1) * (nk / 2) / a.KS) - t.kb;
@@ -649,6 +655,14 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
       __builtin_amdgcn_global_load_lds(
           (const void*)(ws + ((uint32_t)(b >> 1) * kblk + (uint32_t)(b & 1) * 1024u + lw)),
           (lds_void*)((lds_u8*)&wl[st][b * 1024]), 16, 0, 0);
+    }
+  };
+  // the tile's biases: 8 a lane of wave 0, lanes past the tile's columns repeat the last ones
+  auto issue_bias = [&](int n0, int p, int half) {
+    if (BIAS && wave == 0 && a.bias) {
+      const uint32_t last = (uint32_t)(half ? BN / 16 : BN / 8) - 1u;
+      __builtin_amdgcn_global_load_lds((const void*)((const uint8_t*)(a.bias + n0) + 16u * min(gp_lane_now(), last)),
+                                       (lds_void*)((lds_u8*)&bsl[p][0]), 16, 0, 0);
     }
   };
   // Operand reads: x fragment (j, t) = k 32 t + 8 g4 .. +7 of row 128 wm + 16 j + l16, at
@@ -726,6 +740,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
         : "memory");
   };
   Item cur = item_at(0), nxt = item_at(1);
+  issue_bias(cur.n0, 0, cur.half);
   issue(cur.m0, cur.n0, cur.kb, 0, cur.half);
   issue(cur.m0, cur.n0, cur.kb + 1, 1, cur.half);
   gp_wait_vmcnt<XLD + WLD>();           // stage 0
@@ -748,7 +763,10 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
       {
         const int iks = ks + NS;
         if (iks < cur.kc) issue(cur.m0, cur.n0, cur.kb + iks, st, cur.half);
-        else issue(nxt.m0, nxt.n0, nxt.kb + iks - cur.kc, st, nxt.half);
+        else {
+          if (iks == cur.kc) issue_bias(nxt.n0, (r + 1) & 1, nxt.half);
+          issue(nxt.m0, nxt.n0, nxt.kb + iks - cur.kc, st, nxt.half);
+        }
       }
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -795,16 +813,31 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
         };
         pair(acc[0], acc[1], 0);
         if (!cur.half) pair(acc[2], acc[3], 16);
-      } else if constexpr (EPI == GP_STORE) {
+      } else if constexpr (BIAS) {
         half_t* const ob = a.out + mrow + wc + lo;
+        const bool has_bias = a.bias != nullptr;
 #pragma unroll
         for (int i = 0; i < NIW; ++i) {
           if (i >= ni) break;
+          half4_t b = {0, 0, 0, 0};
+          if (has_bias) {
+            // read with its own lgkmcnt wait: the compiler's would also wait for the next
+            // tile's stages in flight
+            typedef __attribute__((address_space(3))) half_t lds_f16;
+            typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+            const uint32_t ab = (uint32_t)(uintptr_t)(lds_f16*)&bsl[r & 1][wc - cur.n0 + 16 * i + 4 * (ln >> 4)];
+            u32x2 bw;
+            asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(bw) : "v"(ab) : "memory");
+            b = __builtin_bit_cast(half4_t, bw);
+          }
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             half4_t o;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = (half_t)acc[i][j][q];
+            for (int q = 0; q < 4; ++q) {
+              const half_t h = gp_bias(acc[i][j][q], b[q], has_bias, a.bias_after_round);
+              o[q] = EPI == GP_QGELU ? gp_quick_gelu(h) : EPI == GP_GELU ? gp_gelu(h) : h;
+            }
             *(half4_t*)(ob + (16 * j * a.ldo + 16 * i)) = o;
           }
         }
@@ -1106,7 +1139,7 @@ static int gp_launch(const GemmPipeArgs& a, int epilogue, hipStream_t st) {
 // [0, 16384) and 192 half tiles over the last 1536); N where no such split exists.
 static int gp_big_tail_cols(int M, int N) {
   const int64_t cus = gp_num_cus();
-  const int64_t tm = M / 256, tn = N / 256;
+  const int64_t tm = ceil_div(M, 256), tn = N / 256;
   const int64_t tiles = tm * tn;
   const int64_t R = tiles / cus;
   if (R == 0 || tiles % cus == 0 || (R * cus) % tm) return N;
@@ -1226,8 +1259,8 @@ extern "C" int omni_f16_gemm_pipe(const void* x, int ldx, const void* w, const v
 
 // omni_packed_gemm_pipe's tiling for a shape: tile rows and columns and K slices, from the
 // caller's tile_rows / ksplit (0: chosen).  128 x 192 and persistent 256 x 256 tiles only
-// where both were chosen; the 256 x 256 ones (fp16 weights, STORE without a bias / SILU, M
-// and N multiples of 256) where rounds of the grid times the tile's cost (per 128 x 128
+// where both were chosen; the 256 x 256 ones (fp16 weights, STORE / QGELU / GELU / SILU, M
+// from 256, N a multiple of 256) where rounds of the grid times the tile's cost (per 128 x 128
 // outputs: GP_BIG_COST, against 1 or GP_WIDE_COST) come out below the other plan's.
 static void gp_packed_plan(int M, int N, int K, int fmt, int epilogue, bool has_bias, int tile_rows,
                            int ksplit, int& rows, int& cols, int& ks) {
@@ -1288,14 +1321,15 @@ static void gp_packed_plan(int M, int N, int K, int fmt, int epilogue, bool has_
     }
     return;
   }
-  if (((epilogue == GP_STORE && !has_bias) || epilogue == GP_SILU) && M % 256 == 0 && N % 256 == 0) {
+  if ((epilogue == GP_STORE || epilogue == GP_QGELU || epilogue == GP_GELU || epilogue == GP_SILU) &&
+      M >= 256 && N % 256 == 0) {
     const int64_t cus = gp_num_cus();
     auto rounds = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
     const double cur = rounds((int64_t)ceil_div(M, rows) * (N / cols)) * (rows * cols) / 16384.0 *
                        (cols == 192 ? GP_WIDE_COST : 1.0);
     // a half-tile tail round (gp_big_tail_cols) measured at 0.65 of a whole one: M = 4096
     // gate_up + SiLU 204.9 against 221.1 us with whole tiles only
-    const int64_t tb = (int64_t)(M / 256) * (N / 256);
+    const int64_t tb = (int64_t)ceil_div(M, 256) * (N / 256);
     const double big = (gp_big_tail_cols(M, N) < N ? (double)(tb / cus) + GP_TAIL_COST : rounds(tb)) *
                        4.0 * GP_BIG_COST;
     if (big < cur) {
@@ -1385,15 +1419,14 @@ static int gp_packed_f16_launch(GemmPipeArgs& a, int epilogue, int tile_rows, in
                                 hipStream_t st) {
   const int M = a.M, N = a.N;
   const int ksplit = a.KS;
-  const bool bias = a.bias != nullptr;
   if (tile_rows == 256 && cols != GP_BN) {     // persistent 8-wave tiles of 256 x cols
-    if (M % 256 || N % cols || (cols == 192 && epilogue == GP_SILU) || (epilogue == GP_STORE && bias) ||
-        (epilogue != GP_SILU && epilogue != GP_PARTIAL && epilogue != GP_STORE))
+    if (M < 256 || N % cols || (cols == 192 && epilogue != GP_PARTIAL) || epilogue == GP_RESID)
       return OMNI_EINVAL;                      // (the plan picks them only where they hold)
-    int64_t t = (int64_t)(M / 256) * (N / cols) * ksplit;
+    const int64_t tm = ceil_div(M, 256);
+    int64_t t = tm * (N / cols) * ksplit;
     if (cols == 256 && ksplit == 1) {
       a.n_big = gp_big_tail_cols(M, N);
-      t = (int64_t)(M / 256) * (a.n_big / 256 + (N - a.n_big) / 128);
+      t = tm * (a.n_big / 256 + (N - a.n_big) / 128);
     }
     const int grid = (int)(t < gp_num_cus() ? t : gp_num_cus());
     const dim3 blk(512);
@@ -1403,10 +1436,12 @@ static int gp_packed_f16_launch(GemmPipeArgs& a, int epilogue, int tile_rows, in
       hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_PARTIAL, 4>), dim3(grid), blk, 0, st, a);
     else if (epilogue == GP_PARTIAL)
       hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_PARTIAL, 3>), dim3(grid), blk, 0, st, a);
-    else if (cols == 256)
-      hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_STORE, 4>), dim3(grid), blk, 0, st, a);
+    else if (epilogue == GP_QGELU)
+      hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_QGELU, 4>), dim3(grid), blk, 0, st, a);
+    else if (epilogue == GP_GELU)
+      hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_GELU, 4>), dim3(grid), blk, 0, st, a);
     else
-      hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_STORE, 3>), dim3(grid), blk, 0, st, a);
+      hipLaunchKernelGGL((gemm_bigp_f16_kernel<GP_STORE, 4>), dim3(grid), blk, 0, st, a);
     OMNI_CHECK_LAUNCH();
     return OMNI_OK;
   }

@@ -1579,3 +1579,40 @@ def test_fp8_prequant_chain(gpu):
     d = (y.cpu().float() - e).abs()
     tol = e.abs() * 2.0 ** -7 + fp8_abs_product(qc, s.cpu(), wq, sw) * 2.0 ** -14
     assert (d <= tol + 1e-6).all(), (d - tol).max().item()
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(4000, 3840, 256, 0), (3872, 5120, 256, 4), (300, 33024, 256, 0),
+                                       (4095, 5120, 384, 5), (2047, 17920, 256, 1)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_f16_big_tiles_ragged_rows(gpu, M, N, K, epi, bias):
+    """The persistent 256-row tiles at row counts off a multiple of 256 (the last row tile
+    repeats up to 255 rows of the one before it) in every epilogue they have (0 STORE, 1 SILU,
+    4 QGELU, 5 GELU; biases staged per tile; tail columns): bit-equal to the 128 x 128 tiles, and nothing written past the rows or the columns."""
+    import ctypes
+    from omniserver_amd._lib import call, lib, ptr, stream
+    if bias and epi == 1:
+        pytest.skip("no bias in this form")
+    r, c, k = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    lib().omni_packed_gemm_pipe_plan(M, N, K, 1, epi, int(bias), 0, 0, ctypes.byref(r),
+                                     ctypes.byref(c), ctypes.byref(k))
+    say(f"f16 big tiles M={M} N={N} K={K} epi={epi} bias={bias} -> {r.value} x {c.value}, {k.value} slices")
+    assert (r.value, c.value, k.value) == (256, 256, 1)
+    w = f16((N, K), 180, 0.05).to(gpu)
+    wp = torch.empty_like(w)
+    call("omni_f16_pack", ptr(w), ptr(wp), K, N, int(epi == 1), stream())
+    x, b = f16((M, K), 181).to(gpu), f16((N,), 182).to(gpu) if bias else None
+    n_out = N // 2 if epi == 1 else N
+
+    def run(tile_rows):
+        out = torch.full((M + 3, n_out + 4), 5.0, device=gpu, dtype=torch.float16)
+        if epi == 1:
+            call("omni_packed_gemm_pipe", ptr(x), K, ptr(wp), None, 1, None, 0, ptr(out), n_out + 4,
+                 M, N, K, epi, tile_rows, 1 if tile_rows else 0, None, stream())
+        else:
+            call("omni_f16_gemm_pipe_packed", ptr(x), K, ptr(wp), ptr(b), None, 0, ptr(out), n_out + 4,
+                 M, N, K, epi, tile_rows, 1 if tile_rows else 0, None, stream())
+        return out
+
+    got, want = run(0), run(128)
+    assert (got[M:] == 5.0).all() and (got[:, n_out:] == 5.0).all()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
