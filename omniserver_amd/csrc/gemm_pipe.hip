@@ -63,10 +63,18 @@ __device__ __forceinline__ void gp_wait_vmcnt() {
 }
 __device__ __forceinline__ void gp_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// h * sigmoid(1.702 h), each step rounded to fp16.  The sigmoid on the bare exp2 and reciprocal
+// instructions: with expf and an IEEE division, about 40 VALU operations a value while the
+// matrix cores wait, the vision tower's fc1 took 88.8 us at 3872 rows, now 75.5; 24.3 and
+// 22.1 at 1024.  t has 11
+// significant bits, so t times the 13-bit head of -log2(e) is exact and the exponent is
+// rounded once; the sigmoid's error before its fp16 rounding (2^-12) stays below 2^-20.
 __device__ __forceinline__ half_t gp_quick_gelu(half_t h) {
 #pragma clang fp contract(off)
   const float t = (float)(half_t)((float)h * 1.702f);
-  const float sg = (float)(half_t)(1.0f / (1.0f + expf(-t)));
+  constexpr float LH = -11818.0f / 8192.0f;            // head of -log2(e)
+  const float e = __builtin_amdgcn_exp2f(fmaf(t, (float)(-1.4426950408889634 - LH), t * LH));
+  const float sg = (float)(half_t)__builtin_amdgcn_rcpf(1.0f + e);
   return (half_t)((float)h * sg);
 }
 
