@@ -362,7 +362,7 @@ int omni_f16_gemm_pipe_splits(int M, int N, int K, int tile_rows);
  * slices [ksplit][M][N] only, into workspace (out and bias unused, NULL), for a consumer
  * that sums them in order (omni_add_rmsnorm_partials, omni_mrope_kv_write_partials).
  * With tile_rows and ksplit both 0 and fp16 weights, shapes whose 128 x 192 tiles (STORE /
- * PARTIAL, N % 192 == 0) or persistent 256 x 256 tiles (STORE / QGELU / GELU / SILU, M >= 256,
+ * PARTIAL, N % 192 == 0) or persistent 256 x 256 tiles (unbiased STORE / SILU, M >= 256,
  * N % 256 == 0) take fewer grid rounds x tile work run those, and 128 x 160 tiles (N % 160
  * == 0: the SILU epilogue at 129-256 rows as five gate|up pairs, STORE with a bias where one
  * round of them covers more CUs than one round of 128-column tiles) where they fill the CUs

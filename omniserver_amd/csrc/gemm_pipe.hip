@@ -539,8 +539,8 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
   gp_wait_vmcnt<0>();                  // drain the clamped tail loads before exit
 }
 
-// Persistent 256 x 256 or 256 x 192 (PARTIAL) tiles for the packed fp16 weights (every
-// epilogue but RESID, M >= 256, N a multiple of the tile width; rows past the last multiple of
+// Persistent 256 x 256 or 256 x 192 (PARTIAL) tiles for the packed fp16 weights (STORE
+// without a bias, QGELU, GELU, SILU and PARTIAL, M >= 256, N a multiple of the tile width; rows past the last multiple of
 // 256 take a tile that ends at row M - 1 and repeats rows of the tile before it: the same
 // bytes written twice, no bound on loads or stores):
 // 8 waves (two per SIMD: 2 along m x 4 along n), each owning a 128 (m) x 16 NIW (n) block,
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
 // tile's biases ride with its first stage into an LDS slot of their own (two, by tile parity):
 // read from global memory in the epilogue they would wait for the next tile's stages.  The
 // vision tower's linears, 256 x 128 tiles / this, us: 1280 -> 5120 + QGELU at 3872 rows 76.9 /
-// 75.5, 2100 52.4 / 46.5, 2852 54 / 49.5; 1280 -> 3840 at 3872 49.4 / 47.2, 2852 47.9 / 42.8;
+// 75.5, 2100 52.4 / 46.5, 2852 54 / 49.5;
 // 5120 -> 5120 + GELU at 2100 165 / 141.6.  Same k order per output as the
 // kernel above within a slice: one-slice results equal its bit for bit.  MI355X, us
 // (256 x 128 or 128 x 192 / this, interleaved, median of 7): M = 4096 gate_up + SiLU
@@ -577,8 +577,9 @@ __device__ __forceinline__ uint32_t gp_lane_now() {
 template <int EPI, int NIW>
 __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
 #pragma clang fp contract(off)
-  constexpr bool BIAS = EPI == GP_STORE || EPI == GP_QGELU || EPI == GP_GELU;
-  static_assert((EPI == GP_PARTIAL && NIW == 3) || ((EPI == GP_PARTIAL || EPI == GP_SILU || BIAS) && NIW == 4),
+  constexpr bool BIAS = EPI == GP_QGELU || EPI == GP_GELU;
+  static_assert((EPI == GP_PARTIAL && NIW == 3) ||
+                    ((EPI == GP_PARTIAL || EPI == GP_SILU || EPI == GP_STORE || BIAS) && NIW == 4),
                 "PARTIAL at 192 or 256 columns, the others at 256");
   constexpr int NS = 2;
   constexpr int BM = 256;               // tile rows
@@ -821,9 +822,9 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
         };
         pair(acc[0], acc[1], 0);
         if (!cur.half) pair(acc[2], acc[3], 16);
-      } else if constexpr (BIAS) {
+      } else if constexpr (EPI == GP_STORE || BIAS) {
         half_t* const ob = a.out + mrow + wc + lo;
-        const bool has_bias = a.bias != nullptr;
+        const bool has_bias = BIAS && a.bias != nullptr;
 #pragma unroll
         for (int i = 0; i < NIW; ++i) {
           if (i >= ni) break;
@@ -1267,7 +1268,7 @@ extern "C" int omni_f16_gemm_pipe(const void* x, int ldx, const void* w, const v
 
 // omni_packed_gemm_pipe's tiling for a shape: tile rows and columns and K slices, from the
 // caller's tile_rows / ksplit (0: chosen).  128 x 192 and persistent 256 x 256 tiles only
-// where both were chosen; the 256 x 256 ones (fp16 weights, STORE / QGELU / GELU / SILU, M
+// where both were chosen; the 256 x 256 ones (fp16 weights, unbiased STORE, QGELU, GELU, SILU, M
 // from 256, N a multiple of 256) where rounds of the grid times the tile's cost (per 128 x 128
 // outputs: GP_BIG_COST, against 1 or GP_WIDE_COST) come out below the other plan's.
 static void gp_packed_plan(int M, int N, int K, int fmt, int epilogue, bool has_bias, int tile_rows,
@@ -1329,7 +1330,8 @@ static void gp_packed_plan(int M, int N, int K, int fmt, int epilogue, bool has_
     }
     return;
   }
-  if ((epilogue == GP_STORE || epilogue == GP_QGELU || epilogue == GP_GELU || epilogue == GP_SILU) &&
+  if (((epilogue == GP_STORE && !has_bias) || epilogue == GP_QGELU || epilogue == GP_GELU ||
+       epilogue == GP_SILU) &&
       M >= 256 && N % 256 == 0) {
     const int64_t cus = gp_num_cus();
     auto rounds = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
@@ -1428,7 +1430,8 @@ static int gp_packed_f16_launch(GemmPipeArgs& a, int epilogue, int tile_rows, in
   const int M = a.M, N = a.N;
   const int ksplit = a.KS;
   if (tile_rows == 256 && cols != GP_BN) {     // persistent 8-wave tiles of 256 x cols
-    if (M < 256 || N % cols || (cols == 192 && epilogue != GP_PARTIAL) || epilogue == GP_RESID)
+    if (M < 256 || N % cols || (cols == 192 && epilogue != GP_PARTIAL) || epilogue == GP_RESID ||
+        (epilogue == GP_STORE && a.bias))
       return OMNI_EINVAL;                      // (the plan picks them only where they hold)
     const int64_t tm = ceil_div(M, 256);
     int64_t t = tm * (N / cols) * ksplit;
