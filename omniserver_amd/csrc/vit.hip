@@ -577,6 +577,9 @@ extern "C" int omni_vit_attention_rows(const void* qkv, int ld, int S, int n_hea
   a.out = (half_t*)out;
   a.ldo = ldo;
   a.scale_log2 = fabsf(scale) * 1.4426950408889634f;
+  // A masked score times 0 would be NaN.  2^-126 weighs the keys as 0 does: fp16 heads' scores
+  // are below 2^40, so every exponent is under 2^-86 and every exp2 exactly 1.
+  if (a.scale_log2 < 0x1p-126f) a.scale_log2 = 0x1p-126f;
   a.negate = scale < 0.f;
   const bool al = (((uintptr_t)qkv | (uintptr_t)out) & 15) == 0 && (ldo & 7) == 0;
   const dim3 gd((unsigned)grid);

@@ -155,6 +155,26 @@ def test_vit_attention_tiles(gpu, segs, step, scale, off):
             assert d <= 4e-3, (a, h, d)
 
 
+@pytest.mark.parametrize("step", [64, 128])
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-42])
+def test_vit_attention_scale_zero(gpu, step, scale):
+    """A scale of zero (or one under the normal range) weighs every key of the segment alike:
+    the mean of V, in segments that end inside a key tile and on one.  Tolerance: the fp16
+    rounding of the output (2^-11 of values below 4) and of the fp32 sums."""
+    from omniserver_amd import vit
+    nh, hd, segs = 3, 80, [70, 64, 5]
+    S = sum(segs)
+    say(f"vit_attention step={step} scale={scale}")
+    qkv = f16((S, 3 * nh * hd), 11).to(gpu)
+    cu = torch.tensor([0, 70, 134, 139], dtype=torch.int32)
+    out = torch.full((S, nh * hd), float("nan"), device=gpu, dtype=torch.float16)
+    vit.vit_attention_out(qkv, nh, hd, cu.to(gpu), vit.query_tiles(cu, step).to(gpu), scale, out, step)
+    v = qkv.cpu().double()[:, 2 * nh * hd:]
+    for a, b in zip(cu.tolist(), cu.tolist()[1:]):
+        d = (out[a:b].cpu().double() - v[a:b].mean(0)).abs().max().item()
+        assert d <= 2.0 ** -9, (a, d)
+
+
 def _tower(gpu, depth, seed):
     from omniserver_amd import synth, vit
     cfg = vit.VisionConfig(depth=depth)
