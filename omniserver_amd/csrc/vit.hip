@@ -350,8 +350,9 @@ struct VitAttnArgs {
   int negate;          // the scale was negative: its sign goes to q
 };
 
-// ALIGNED: qkv and out on 16-byte boundaries, ldo a multiple of 8 (tiles straight to LDS,
-// 16-byte stores); otherwise staged through registers and stored by element.
+// ALIGNED: qkv and out on 16-byte boundaries, ldo a multiple of 8, ld within the 32-bit lane
+// offsets (tiles straight to LDS, 16-byte stores); otherwise staged through registers and stored
+// by element.
 template <int R, int S, int KT, bool ALIGNED>
 __global__ __launch_bounds__(64 * R * S, 2) void vit_attn_kernel(VitAttnArgs a) {
   constexpr int NB = KT / 32;
@@ -415,11 +416,12 @@ __global__ __launch_bounds__(64 * R * S, 2) void vit_attn_kernel(VitAttnArgs a) 
     for (int i = 0; i < NW; ++i) {
       const int J = rt + R * i;
       if (NI % R && J >= NI) continue;
-      const uint32_t off = (uint32_t)min(prow[i], last) * (uint32_t)a.ld * 2 + psrc[i];
       if constexpr (ALIGNED)
-        dma16(src, off, __builtin_amdgcn_readfirstlane(lds_offset(dst)) + 1024 * J);
+        dma16(src, (uint32_t)min(prow[i], last) * (uint32_t)a.ld * 2 + psrc[i],
+              __builtin_amdgcn_readfirstlane(lds_offset(dst)) + 1024 * J);
       else
-        *(half8_t*)(dst + 1024 * J + 16 * lane) = *(const half8_t*)((const char*)src + off);
+        *(half8_t*)(dst + 1024 * J + 16 * lane) =
+            *(const half8_t*)((const char*)(src + (int64_t)min(prow[i], last) * a.ld) + psrc[i]);
     }
   };
 
@@ -581,7 +583,8 @@ extern "C" int omni_vit_attention_rows(const void* qkv, int ld, int S, int n_hea
   // are below 2^40, so every exponent is under 2^-86 and every exp2 exactly 1.
   if (a.scale_log2 < 0x1p-126f) a.scale_log2 = 0x1p-126f;
   a.negate = scale < 0.f;
-  const bool al = (((uintptr_t)qkv | (uintptr_t)out) & 15) == 0 && (ldo & 7) == 0;
+  // a staged tile spans 64 rows of 2 ld bytes: below 2^32 up to ld = 2^24
+  const bool al = (((uintptr_t)qkv | (uintptr_t)out) & 15) == 0 && (ldo & 7) == 0 && ld <= 1 << 24;
   const dim3 gd((unsigned)grid);
   hipStream_t st = (hipStream_t)stream;
   const dim3 bd(512);

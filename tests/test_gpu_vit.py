@@ -175,6 +175,32 @@ def test_vit_attention_scale_zero(gpu, step, scale):
         assert d <= 2.0 ** -9, (a, d)
 
 
+@pytest.mark.parametrize("step", [64, 128])
+def test_vit_attention_wide_rows(gpu, step):
+    """Rows 2^25 + 8 halfs apart (a view into a wide buffer): the 64 rows of a key tile span
+    more than 32 bits of byte offsets.  Bit-equal to the same rows packed but 8 bytes off the
+    16-byte boundary, the form without 32-bit offsets."""
+    from omniserver_amd import vit
+    from omniserver_amd._lib import call, ptr, stream
+    nh, hd, S, ld = 1, 80, 130, 2 ** 25 + 8
+    w = 3 * nh * hd
+    say(f"vit_attention wide rows step={step}")
+    x = f16((S, w), 12).to(gpu)
+    wide = torch.empty((S - 1) * ld + w, device=gpu, dtype=torch.float16)
+    wide.as_strided((S, w), (ld, 1)).copy_(x)
+    off = torch.empty(S * w + 8, device=gpu, dtype=torch.float16)[4:4 + S * w].view(S, w).copy_(x)
+    cu = torch.tensor([0, S], dtype=torch.int32)
+    tiles, cu_g = vit.query_tiles(cu, step).to(gpu), cu.to(gpu)
+    outs = []
+    for t, stride in ((wide, ld), (off, w)):
+        out = torch.full((S, nh * hd), float("nan"), device=gpu, dtype=torch.float16)
+        call("omni_vit_attention_rows", ptr(t), stride, S, nh, hd, ptr(cu_g), ptr(tiles),
+             tiles.shape[0], ptr(out), nh * hd, hd ** -0.5, step, stream())
+        outs.append(out)
+    assert not torch.isnan(outs[1]).any()
+    assert torch.equal(outs[0], outs[1])
+
+
 def _tower(gpu, depth, seed):
     from omniserver_amd import synth, vit
     cfg = vit.VisionConfig(depth=depth)
