@@ -1429,6 +1429,13 @@ static int gp_packed_f16_launch(GemmPipeArgs& a, int epilogue, int tile_rows, in
                                 hipStream_t st) {
   const int M = a.M, N = a.N;
   const int ksplit = a.KS;
+  // The persistent 256 x 256 / 192 tiles address 255 rows by 32-bit offsets: rows up to 2^22
+  // elements apart.  Wider ones take the 256 x 128 tiles (64-bit addresses, the same sums),
+  // whose three stages need as many steps per slice.
+  if (tile_rows == 256 && cols != GP_BN && (a.ldx > 1 << 22 || a.ldo > 1 << 22)) {
+    if (2 * (a.K / 128 / ksplit) < 3) return OMNI_EUNSUPPORTED;
+    cols = GP_BN;
+  }
   if (tile_rows == 256 && cols != GP_BN) {     // persistent 8-wave tiles of 256 x cols
     if (M < 256 || N % cols || (cols == 192 && epilogue != GP_PARTIAL) || epilogue == GP_RESID ||
         (epilogue == GP_STORE && a.bias))

@@ -1616,3 +1616,27 @@ def test_f16_big_tiles_ragged_rows(gpu, M, N, K, epi, bias):
     got, want = run(0), run(128)
     assert (got[M:] == 5.0).all() and (got[:, n_out:] == 5.0).all()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("epi,ldx,ldo", [(0, 2 ** 23 + 8, 33024), (0, 256, 2 ** 25 + 4),
+                                         (5, 2 ** 23 + 8, 2 ** 22 + 4)])
+def test_f16_big_tiles_wide_rows(gpu, epi, ldx, ldo):
+    """Shapes of the persistent 256 x 256 tiles whose rows are further apart than their 32-bit
+    offsets reach (a view into a wide buffer): bit-equal to the same call on packed rows."""
+    from omniserver_amd._lib import call, ptr, stream
+    M, N, K = 300, 33024, 256
+    say(f"f16 big tiles wide rows epi={epi} ldx={ldx} ldo={ldo}")
+    w = f16((N, K), 183, 0.05).to(gpu)
+    wp = torch.empty_like(w)
+    call("omni_f16_pack", ptr(w), ptr(wp), K, N, 0, stream())
+    x = f16((M, K), 184).to(gpu)
+
+    def run(lx, lo):
+        xb = torch.empty((M - 1) * lx + K, device=gpu, dtype=torch.float16)
+        xb.as_strided((M, K), (lx, 1)).copy_(x)
+        ob = torch.empty((M - 1) * lo + N, device=gpu, dtype=torch.float16)
+        call("omni_f16_gemm_pipe_packed", ptr(xb), lx, ptr(wp), None, None, 0, ptr(ob), lo, M, N,
+             K, epi, 0, 1, None, stream())
+        return ob.as_strided((M, N), (lo, 1)).clone()
+
+    assert torch.equal(run(ldx, ldo).view(torch.int16), run(K, N).view(torch.int16))
