@@ -504,7 +504,8 @@ int omni_fp8_gemm_plan(int M, int N, int K, int* grid);
  * as out_mode stores them (no bias), in the same type; bit-equal to omni_fp8_gemm +
  * omni_silu_mul(_bf16).  amax_part (may be NULL): omni_fp8_gemm_silu_grid floats, partial maxima
  * of |out| for omni_fp8_quant_tensor_parts.  -2 where the grid is 0: M < 256,
- * K < 1024, N not a multiple of 256, or shapes the two launches are faster for. */
+ * K < 1024, N not a multiple of 256, or shapes the two launches are faster for; and for
+ * ldo > 2^22. */
 int omni_fp8_gemm_silu(const void* xq, const float* sa, const void* wq, const float* sw, void* out,
                        int ldo, float* amax_part, int M, int N, int K, int out_mode, void* stream);
 int omni_fp8_gemm_silu_grid(int M, int N, int K);

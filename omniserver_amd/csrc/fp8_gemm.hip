@@ -493,6 +493,9 @@ __global__ __launch_bounds__(128 * WM, 1) void fp8_gemm_pipe_kernel(Fp8GemmArgs 
 // column tiles, so M = 8192 gives 256 tiles, one per CU, where the 256-column tiles leave a
 // quarter of the CUs idle.
 #define F8B_T 256
+// Their epilogue steps through a wave's 128 output rows by 32-bit offsets; rows further apart
+// take the 256 x 128 tiles' 64-bit addresses (the SiLU form: refused).
+#define F8B_MAX_LDO (1 << 22)
 
 // Two adjacent product values v = acc * sa * sw stored, packed (v0 low), in out_mode's form:
 // bf16(v) plus bf16(bias) as a bf16 add (FP8_OUT_BF16: forward_prequant, out + bias.to(bf16)),
@@ -1365,7 +1368,7 @@ extern "C" int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, co
   a.K = K;
   a.out_mode = out_mode;
   a.n_big = N;
-  const int bc = fp8_big_cols(M, N, K);
+  const int bc = ldo <= F8B_MAX_LDO ? fp8_big_cols(M, N, K) : 0;
   if (bc) {                                       // persistent 256 x bc tiles
     if (bc == 256) a.n_big = fp8_tail_cols(M, N);
     const int64_t bt = fp8_big_items(M, N, bc);
@@ -1425,7 +1428,7 @@ extern "C" int omni_fp8_gemm_silu(const void* xq, const float* sa, const void* w
   if (out_mode < FP8_OUT_F16_VIA_BF16 || out_mode > FP8_OUT_F16) return OMNI_EINVAL;
   if (M == 0) return OMNI_OK;
   const int grid = omni_fp8_gemm_silu_grid(M, N, K);
-  if (!grid) return OMNI_EUNSUPPORTED;
+  if (!grid || ldo > F8B_MAX_LDO) return OMNI_EUNSUPPORTED;
   if (ldo < N / 2 || (ldo & 3)) return OMNI_EINVAL;
   if (!xq || !sa || !wq || !sw || !out) return OMNI_EINVAL;
   if (((uintptr_t)xq & 15) || ((uintptr_t)wq & 15) || ((uintptr_t)sa & 3) || ((uintptr_t)sw & 3) ||

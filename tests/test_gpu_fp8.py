@@ -184,3 +184,27 @@ def test_fp8_few_rows(gpu, M, K, N, bias):
         tol = mag * 2.0 ** -14 + (eps + 2.0 ** -11) * (2 * v.abs() + 2 * bb.abs()) + 1e-6
         assert (d <= tol).all(), (mode, (d - tol).max().item())
         assert (buf[:, N:] == 5.0).all()
+
+
+@pytest.mark.parametrize("ldo", [2 ** 22 + 4, 2 ** 25 + 4])
+def test_fp8_big_tiles_wide_rows(gpu, ldo):
+    """A ragged shape of the big tiles whose output rows are further apart than their 32-bit
+    offsets reach: bit-equal to the same product in packed rows, in every output form; the
+    SiLU form refuses such rows."""
+    from omniserver_amd._lib import lib, ptr, stream
+    from omniserver_amd.linear import FP8Linear
+    M, N, K = 300, 36864, 1024
+    assert plan(M, N, K)[0] in (2, 3)
+    say(f"fp8 big tiles wide rows ldo={ldo}")
+    lin = FP8Linear(f16((N, K), 420, 0.02).to(gpu), f16((N,), 421).to(gpu), rowwise=True)
+    xq, sa = lin.quantize_input(f16((M, K), 422).to(gpu))
+    buf = torch.empty((M - 1) * ldo + N, device=gpu, dtype=torch.float16)
+    for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16, lin.OUT_F16):
+        dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
+        wide = buf.view(dt).as_strided((M, N), (ldo, 1))
+        lin.gemm_out(xq, sa, wide, mode)
+        want = lin.gemm_out(xq, sa, torch.empty(M, N, device=gpu, dtype=dt), mode)
+        assert torch.equal(wide.contiguous().view(torch.int16), want.view(torch.int16)), mode
+    assert lib().omni_fp8_gemm_silu_grid(M, N, K) > 0
+    assert lib().omni_fp8_gemm_silu(ptr(xq), ptr(sa), ptr(lin.weight_fp8), ptr(lin.weight_scale),
+                                    ptr(buf), ldo, None, M, N, K, lin.OUT_BF16, stream()) == -2
