@@ -13,7 +13,7 @@ of workgroups and the longest context (``prefill_plan``):
   kernel's longer start and merge show;
 * omni_prefill_attention (one wave per item) and its split form, whose accesses ask for no
   alignment, for what the rows kernel does not take: more than 32 query heads per KV head,
-  scale <= 0, operands off a 16-byte boundary.
+  a scale that is not a positive normal fp32, operands off a 16-byte boundary.
 
 MI355X, 12 heads / 2 KV heads, us per launch, rows (128, 1) / (128, 2) / (64, 4) / (32, 8),
 then the best of the per-wave, split and shared-tile kernels: one 4096-token prompt 86.8 /
@@ -109,7 +109,8 @@ def prefill_attention_pool(writer, q: torch.Tensor, layer_idx: int, scale: float
     if plans is None:
         plans = writer._attn_plan = {}
     qp, op = q.data_ptr(), out.data_ptr()
-    plain = bool((qp | op) & 15) or not scale > 0
+    # also a scale that fp32 does not hold as a normal number, which the rows kernel refuses
+    plain = bool((qp | op) & 15) or not scale >= 2.0 ** -126
     plan = plans.get(plain)
     if plan is None:
         cus = num_cus(q.device)

@@ -351,6 +351,23 @@ def test_prefill_attention_pool_unaligned(gpu):
     assert (outs[0] - outs[1]).abs().max().item() <= 4e-3
 
 
+@pytest.mark.parametrize("scale", [0.0, 1e-60, 1e-42])
+def test_prefill_attention_pool_scale_zero(gpu, scale):
+    """A scale that fp32 holds as zero or as a subnormal weighs all visible keys alike.
+    Tolerance: the fp16 rounding of the output (values below 4) and the fp32 sums."""
+    from omniserver_amd.attention import prefill_attention_pool
+    from omniserver_amd.kv_cache import PreallocatedKVCache
+    say(f"prefill_attention_pool scale={scale}")
+    pool = PreallocatedKVCache(1, 2, 2, 512, 128, gpu, n_heads=12)
+    pool.storage.copy_(f16(tuple(pool.storage.shape), 72))
+    w = pool.mixed_cache([0, 1], [300, 70], [100, 0])
+    out = torch.empty(370, 12, 128, device=gpu, dtype=torch.float16)
+    prefill_attention_pool(w, f16((370, 12 * 128), 73).to(gpu), 0, scale, out)
+    mean = pool.v[0].double().cumsum(1) / torch.arange(1, 513, device=gpu).view(1, -1, 1, 1)
+    want = torch.cat([mean[0, 100:400], mean[1, :70]]).repeat_interleave(6, 1)
+    assert (out.double() - want).abs().max().item() <= 2.0 ** -9
+
+
 # ----------------------------------------------------------------------------- linears
 def _gptq(K, N, seed):
     from omniserver_amd.synth import gptq_random
