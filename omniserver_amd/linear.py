@@ -710,7 +710,8 @@ class FP8Linear(nn.Module):
         """fp16 or bf16 x (the bf16 silu_mul output of the fused FP8 MLP route,
         qwen2_llm.py:132-134) -> fp16.  ``amax_parts``: see quantize_input."""
         x2d = self._rows(x)
-        xq, sa = self.quantize_input(x2d, amax_parts)
+        xq, sa = (self.quantize_input(x2d) if amax_parts is None
+                  else self.quantize_input(x2d, amax_parts))
         out = torch.empty(x2d.shape[0], self.N, device=x.device, dtype=torch.float16)
         self.gemm_out(xq, sa, out, self.OUT_F16_VIA_BF16 if self.rowwise else self.OUT_F16)
         return out.reshape(*x.shape[:-1], self.N)

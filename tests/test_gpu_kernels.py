@@ -1460,6 +1460,72 @@ def test_fp8_mlp_fused_silu(gpu, M, rowwise):
     assert seen == [(M, 17920), 1]
 
 
+@pytest.mark.parametrize("prequant", [False, True])
+def test_fp8_mlp_calls_stay_visible(gpu, prequant, monkeypatch):
+    """At a size where the FP8 MLP fuses its launches, whatever watches or replaces its linears'
+    calls still does, with the arguments and results of the unfused calls: hooks on all
+    modules, a subclass or an instance with its own gemm_out or one-argument quantize_input, a
+    method replaced on the class, a gate_up that says it has applied the SiLU itself."""
+    from torch.nn.modules import module as M
+    from omniserver_amd import fused_ops as F
+    from omniserver_amd._lib import lib
+    from omniserver_amd.linear import FP8Linear
+    from omniserver_amd.qwen2_llm import MLP
+    rows = 300
+    say(f"fp8 mlp visible calls prequant={prequant}")
+    gu = FP8Linear(f16((17920, 1536), 174, 0.05).to(gpu), rowwise=prequant)
+    down = FP8Linear(f16((1536, 8960), 175, 0.05).to(gpu))
+    x = f16((rows, 1536), 176).to(gpu)
+    assert lib().omni_fp8_gemm_silu_grid(rows, gu.N, gu.K) > 0
+    if prequant:
+        x = gu.quantize_input(x)
+        x = (x[0].view(torch.float8_e4m3fn), x[1])
+    mlp = MLP(gu, down)
+    product = gu.forward_prequant(*x) if prequant else gu(x)
+    want = down(F.silu_mul(product))
+    same = lambda: torch.equal(mlp(x), want)
+    assert same()
+
+    seen = []
+    calls = [("down", 1)] if prequant else [("gate_up", 1), ("down", 1)]
+    name = lambda m: "gate_up" if m is gu else "down" if m is down else None
+    for reg in (M.register_module_forward_hook, M.register_module_forward_pre_hook):
+        h = reg(lambda m, args, *out: name(m) and seen.append((name(m), len(args))))
+        assert same() and seen == calls
+        h.remove(), seen.clear()
+
+    class Own(FP8Linear):
+        def gemm_out(self, xq, sa, out, mode):
+            seen.append("gemm_out")
+            return super().gemm_out(xq, sa, out, mode)
+
+        def quantize_input(self, x2d):
+            seen.append("quantize_input")
+            return super().quantize_input(x2d)
+
+    for lin in (gu, down):
+        lin.__class__ = Own
+        assert same()
+        assert seen == ["gemm_out"] if prequant and lin is gu else ["quantize_input", "gemm_out"]
+        lin.__class__ = FP8Linear
+        seen.clear()
+        lin.gemm_out = lambda *a, lin=lin: (seen.append("set"), FP8Linear.gemm_out(lin, *a))[1]
+        assert same() and seen == ["set"]
+        del lin.gemm_out
+        seen.clear()
+    for method in ("gemm_out", "forward_prequant" if prequant else "forward"):
+        own = getattr(FP8Linear, method)
+        with monkeypatch.context() as mp:
+            mp.setattr(FP8Linear, method, lambda self, *a, own=own: (seen.append(self), own(self, *a))[1])
+            assert same() and gu in seen
+        seen.clear()
+    square = FP8Linear(f16((1536, 1536), 177, 0.05).to(gpu), rowwise=prequant)
+    square.fuse_silu = True
+    out = square.forward_prequant(*x) if prequant else square(x)
+    last = FP8Linear(f16((1536, 1536), 178, 0.05).to(gpu))
+    assert torch.equal(MLP(square, last)(x), last(out))
+
+
 def fp8_abs_product(xq, sa, wq, sw):
     """|xq| . |wq|^T * sa * sw: the scale of the terms each output sums."""
     return (xq.float().abs() @ wq.float().abs().t()) * sa.view(-1, 1) * sw.view(1, -1)
