@@ -25,6 +25,7 @@ weight format and shape; the decode step of the 2B decoder uses the entries belo
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Dict, Tuple
 
 import torch
@@ -100,6 +101,43 @@ def _unpack_scratch(device: torch.device, halfs: int) -> torch.Tensor:
     return buf
 
 
+# What the skinny kernels stage of x in LDS at most (launch_gemv's limit)
+_SKINNY_X_LDS = 160 * 1024 - 4096
+
+
+@functools.lru_cache(maxsize=4096)
+def _skinny_plan(fmt: str, K: int, N: int, M: int):
+    """(K slices, preset; None: the linear's store preset) of a finished linear without the SiLU
+    epilogue at M <= MAX_SKINNY_M rows; 1 slice: one launch of the store kernel.  Its preset 2
+    gives a workgroup 64 columns, which at N = 1536 makes 24 of them, and stages all of K's x
+    in LDS, past whose size it crawls.  Preset 4 gives 16 columns, K over the 8 waves: while
+    those fit one round of 256 workgroups it wins until each has much x to read (rows x K);
+    beyond that fp32 slices over the grid and a finish launch.  MI355X, us in a graph, weights
+    from memory (preset 2 / 4 / split): int4 1536 -> 1536 M = 1 5.4 / 3.8 / 6.8, 32 7.2 / 5.8 /
+    8.2, 64 25.8 / 9.6 / 9.3; 8960 -> 1536 M = 1 23.7 / 9.9 / 10.0, 12 32.6 / 11.7 / 10.5, 16
+    38.0 / 12.9 / 11.2, 17 45.1 / 15.2 / 11.3, 64 131 / 36.4 / 15.9; 3584 -> 3584 M = 32 29.5 /
+    10.3 / 10.9, 48 42.0 / 13.7 / 12.2; 18944 -> 3584 M = 1 49.8 / 19.0 / 23.0, 16 76.7 / 24.6 /
+    24.8; 4992 -> 4608 M = 1 15.6 / 10.4 / 9.7; fp16 1536 -> 1536 M = 1 7.4 / 4.4 / 7.2, 32 9.0 /
+    6.4 / 8.7; 8960 -> 1536 M = 1 36.3 / 15.4 / 13.3, 16 50.3 / 17.7 / 15.0, 64 144 / 41.2 / 18.5;
+    3584 -> 3584 M = 32 35.3 / 12.8 / 12.8, 48 47.8 / 16.2 / 14.0; 18944 -> 3584 M = 1 80.2 / 34.5 /
+    40.0, 24 145 / 46.2 / 46.6, 32 174 / 52.0 / 47.8.  The line lies where calls outside a graph
+    put it, since the captured step takes the partial form: a split costs 12 us of host time
+    there, one launch 6.5, and the MLP half at one fp16 row 39.2 us against 33.5, so preset 4
+    keeps the up to 2.7 us that a graph would give back below 16 rows of K = 8960.  Rows count
+    by whole blocks past the first.  Slices: 7 groups each (int4), 3.5 (fp16, four times the
+    bytes), from the same sweeps."""
+    KG, padded = K // 128, -(-M // 16) * 16
+    if KG < 4:
+        return 1, None
+    if N // 16 <= 256:
+        if (M if M <= 16 else padded) * KG <= 1152:
+            return 1, 4
+    elif padded * (K + 8) * 2 <= _SKINNY_X_LDS or N // 64 >= 256:
+        return 1, None
+    ks = min(KG, max(6, KG * (1 if fmt == "int4" else 2) // 7))
+    return ks, 3 if KG >= 24 and N % 32 == 0 else 1
+
+
 class _Skinny(nn.Module):
     """Shared launch logic of the packed-weight linears."""
 
@@ -140,34 +178,12 @@ class _Skinny(nn.Module):
             return max(1, min(KG // 2, 256 // tiles))
         return max(1, min(8, KG // 4, 256 // tiles))
 
-    # K slices per 128-group of the finished skinny form where it splits, and the fewest
-    SKINNY_SLICES, SKINNY_MIN_SLICES = (2, 7), 6
-
     def skinny_plan(self, M: int) -> Tuple[int, int]:
-        """(K slices, preset) of the finished form at up to MAX_SKINNY_M rows; 1 slice: one
-        launch of the store kernel.  Its preset 2 gives a workgroup 64 columns, which at
-        N = 1536 makes 24 of them, and stages all of K's x in LDS, past whose size it crawls.
-        Preset 4 gives 16 columns, K over the 8 waves: while those fit one round of 256
-        workgroups it wins until each has much x to read (rows x K); beyond that fp32 slices
-        over the grid and a finish launch.  MI355X, graph-timed, us (preset 2 / 4 / split):
-        int4 1536 -> 1536 M = 1 5.6 / 4.1 / 6.6, 32 6.8 / 5.8 / 8.0, 64 25.8 / 9.7 / 9.2;
-        8960 -> 1536 M = 1 23.9 / 10.1 / 10.2, 16 38 / 13.2 / 11.3, 32 68 / 20.9 / 12.3, 64 132 /
-        - / 15.8; 3584 -> 3584 M = 32 29.8 / 10.4 / 10.7, 48 42.1 / 13.8 / 12.3; 3584 -> 4608
-        M = 1 9.4 / 10.0 / 9.0, 32 29.6 / 17.1 / 11.3; 1536 -> 8960 M = 48 10.1 / 19.4 / 13.6;
-        fp16 1536 -> 1536 M = 1 7.6 / 4.6 / 7.5, 32 9.2 / 6.8 / 8.7; 8960 -> 1536 M = 1 36.7 /
-        15.7 / 13.6, 32 81 / 25.3 / 15.8, 64 144 / - / 18.6.  Slices: 7 groups each (int4), 3.5
-        (fp16, four times the bytes), from the same sweeps."""
-        KG, blocks = self.K // 128, -(-M // 16)
-        if self.fuse_silu or KG < 4:
+        """(K slices, preset) of the finished form at up to MAX_SKINNY_M rows, see _skinny_plan."""
+        if self.fuse_silu:
             return 1, self.store_preset
-        if self.N // 16 <= 256:
-            if blocks * KG <= 72:
-                return 1, 4
-        elif blocks * 16 * (self.K + 8) * 2 <= 160 * 1024 or self.N // 64 >= 256:
-            return 1, self.store_preset
-        num, den = self.SKINNY_SLICES
-        ks = min(KG, max(self.SKINNY_MIN_SLICES, KG * num // den))
-        return ks, 3 if KG >= 24 and self.N % 32 == 0 else 1
+        ks, preset = _skinny_plan(self.fmt, self.K, self.N, M)
+        return ks, self.store_preset if preset is None else preset
 
     def forward_out(self, x2d: torch.Tensor, out: torch.Tensor, preset: int | None = None,
                     ksplit: int | None = None):
@@ -176,8 +192,8 @@ class _Skinny(nn.Module):
         along K as tile_ksplit says unless ``ksplit`` is given)."""
         epi = EPI_SILU if self.fuse_silu else EPI_STORE
         M = x2d.shape[0]
-        if 0 < M <= MAX_SKINNY_M and preset is None and ksplit is None:
-            ks, pr = self.skinny_plan(M)
+        if 0 < M <= MAX_SKINNY_M and not self.fuse_silu and preset is None and ksplit is None:
+            ks, pr = _skinny_plan(self.fmt, self.K, self.N, M)
             if ks == 1:
                 preset = pr
             elif not ((out.data_ptr() & 7) or (out.stride(0) & 3)):
@@ -337,7 +353,6 @@ class GPTQLinear(_Skinny):
     """W4A16 GPTQ linear: y = fp16(x . dequant(W)) (+ bias, added after rounding)."""
 
     fmt = "int4"
-    SKINNY_SLICES = (1, 7)
 
     def __init__(self, qweight: torch.Tensor, scales: torch.Tensor, bias=None,
                  group_size: int = 128, fuse_silu: bool = False):

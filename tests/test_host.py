@@ -438,3 +438,38 @@ def test_prefill_plan_covers_every_call():
             if group > 32:
                 assert (fn, block, extra) == fallback_plan(segs, nkv * group, 256)
     assert len(forms) == 4
+
+
+def test_skinny_plan():
+    """The finished few-row linears' forms at the edges of their rule: 16-column workgroups
+    (preset 4) up to 1152 rows x K groups (rows in whole blocks past the first), K slices and a
+    finish beyond, the store preset for many columns whose x fits the LDS the kernel stages
+    (160 KiB less 4 KiB) and for short K."""
+    from omniserver_amd.linear import _skinny_plan as plan
+    for fmt, s8960, s3584, s18944 in (("int4", 10, 6, 21), ("fp16", 20, 8, 42)):
+        assert plan(fmt, 8960, 1536, 16) == (1, 4) and plan(fmt, 8960, 1536, 17) == (s8960, 3)
+        assert plan(fmt, 3584, 3584, 32) == (1, 4) and plan(fmt, 3584, 3584, 33) == (s3584, 3)
+        assert plan(fmt, 18944, 3584, 7) == (1, 4) and plan(fmt, 18944, 3584, 8) == (s18944, 3)
+        assert plan(fmt, 1536, 2048, 64) == (1, 4)
+        # 4096 < N < 16384: x of one, two and three row blocks in and past the LDS
+        assert plan(fmt, 4864, 4608, 16) == (1, None) and plan(fmt, 4992, 4608, 1)[0] > 1
+        assert plan(fmt, 2432, 4608, 32) == (1, None) and plan(fmt, 2560, 4608, 17)[0] > 1
+        assert plan(fmt, 1536, 4608, 48) == (1, None) and plan(fmt, 1664, 4608, 33)[0] > 1
+        assert plan(fmt, 8960, 16384, 64) == (1, None)
+        assert plan(fmt, 384, 1536, 64) == (1, None)
+        assert plan(fmt, 512, 16, 64) == (1, 4)
+        assert plan(fmt, 8960, 1552, 64)[1] == 1          # N off the 32 columns of preset 3
+        for M in (1, 16, 17, 64):
+            for K in (512, 1536, 8960):
+                assert 1 <= plan(fmt, K, 1536, M)[0] <= K // 128
+
+
+def test_skinny_plan_follows_store_preset():
+    from types import SimpleNamespace
+    from omniserver_amd.linear import _Skinny
+    lin = SimpleNamespace(fmt="int4", K=1536, N=4608, fuse_silu=False, store_preset=2)
+    assert _Skinny.skinny_plan(lin, 8) == (1, 2)
+    lin.store_preset = 0
+    assert _Skinny.skinny_plan(lin, 8) == (1, 0)
+    lin.fuse_silu = True
+    assert _Skinny.skinny_plan(lin, 8) == (1, 0)
