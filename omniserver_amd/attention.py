@@ -29,6 +29,9 @@ keys 78.3 / 61.0 / 46.4 / 56.1, 107; 32 single tokens at 2048 keys 40.8 / 33.1 /
 
 from __future__ import annotations
 
+import operator
+from array import array
+
 import torch
 
 from ._lib import call, ptr, stream
@@ -52,14 +55,33 @@ def num_cus(device) -> int:
 
 
 def query_blocks(seg_lengths, device, block: int = QBLOCK) -> torch.Tensor:
-    """int32 [nqb, 2] (first token, count) covering every segment in blocks of <= block."""
-    blocks = []
+    """int32 [nqb, 2] (first token, count) covering every segment in blocks of <= block.  Built
+    a segment at a time: on a new ragged batch it is part of the first layer's call."""
+    first, count = [], []
     off = 0
     for L in seg_lengths:
-        for s in range(0, L, block):
-            blocks.append((off + s, min(block, L - s)))
+        first += range(off, off + L, block)
+        whole, rest = divmod(L, block)
+        count += [block] * whole
+        if rest:
+            count.append(rest)
         off += L
-    return to_device(blocks, torch.int32, device).reshape(-1, 2)
+    table = [0] * (2 * len(first))
+    table[::2], table[1::2] = first, count
+    if not table:
+        return torch.empty(0, 2, dtype=torch.int32, device=device)
+    return to_device(torch.frombuffer(array("i", table), dtype=torch.int32), torch.int32,
+                     device).view(-1, 2)
+
+
+def _blocks_fit(seg_lengths, tokens: int, block: int, most: int) -> bool:
+    """Whether blocks of at most block tokens cover the segments (tokens in all) in at most
+    most of them; counted only where the sum and number of segments leave it open."""
+    if -(-tokens // block) > most:
+        return False
+    if tokens // block + len(seg_lengths) <= most:
+        return True
+    return sum([-(-L // block) for L in seg_lengths]) <= most
 
 
 def prefill_plan(seg_lengths, starts, nh: int, nkv: int, cus: int) -> tuple:
@@ -67,26 +89,26 @@ def prefill_plan(seg_lengths, starts, nh: int, nkv: int, cus: int) -> tuple:
     tokens appended at starts, in 16-byte aligned tensors (see the module docstring for what
     each form measures)."""
     group = nh // nkv
-    blocks = lambda n: sum(-(-L // n) for L in seg_lengths)
-    wgs = lambda rows: blocks(rows // group) * nkv
-    keys = max(st + L for st, L in zip(starts, seg_lengths))
-    items = blocks(QBLOCK) * nh
     if group > ROWS_MAX_GROUP:
         return fallback_plan(seg_lengths, nh, cus)
+    tokens = sum(seg_lengths)
+    keys = max(map(operator.add, starts, seg_lengths), default=0)
+    items_fit = lambda most: _blocks_fit(seg_lengths, tokens, QBLOCK, most // nh)
+    wgs_fit = lambda rows, most: _blocks_fit(seg_lengths, tokens, rows // group, most // nkv)
     # A few short contexts: the split kernel starts and merges in 2-3 us less (1 x 256: 6.5
     # against 7.5 us, 16 x 24: 4.5 against 6.5) until its items queue (2 x 256: 9.0 against
     # 7.6) or the keys are many (a 128-token chunk at 500 keys: level).
-    if (keys <= 320 and items <= cus) or (keys <= 64 and items <= 2 * cus):
+    if keys <= 320 and items_fit(cus if keys > 64 else 2 * cus):
         return ("omni_prefill_attention_split", QBLOCK, ())
     # Rows to spare for every CU only in 128s: fewer rows per workgroup while those still fit
     # one round of the CUs, with the keys dealt to as many groups as the waves allow.  A long
     # context takes 64 rows also where they are more than one round but 128 would leave CUs
     # idle: the last blocks' chain of key tiles is what counts (1 x 2048: 29.1 against 34.9).
-    if wgs(32) <= cus:
+    if wgs_fit(32, cus):
         form = (32, 8)
-    elif wgs(64) <= cus or (wgs(128) < cus and keys >= 1024):
+    elif wgs_fit(64, cus) or (keys >= 1024 and wgs_fit(128, cus - 1)):
         form = (64, 4)
-    elif keys > 1024 and wgs(128) < 4 * cus:
+    elif keys > 1024 and wgs_fit(128, 4 * cus - 1):
         form = (128, 2)      # 2 x 2048: 39.7 against 54.8 us in one group
     else:
         form = (128, 1)      # short chains, or workgroups enough: 8 x 512 22.6 against 24.4
@@ -95,8 +117,7 @@ def prefill_plan(seg_lengths, starts, nh: int, nkv: int, cus: int) -> tuple:
 
 def fallback_plan(seg_lengths, nh: int, cus: int) -> tuple:
     """The kernels that take any head grouping, scale sign and operand alignment."""
-    items = sum(-(-L // QBLOCK) for L in seg_lengths) * nh
-    split = items <= SPLIT_ITEMS_PER_CU * cus
+    split = _blocks_fit(seg_lengths, sum(seg_lengths), QBLOCK, SPLIT_ITEMS_PER_CU * cus // nh)
     return ("omni_prefill_attention_split" if split else "omni_prefill_attention", QBLOCK, ())
 
 

@@ -473,3 +473,24 @@ def test_skinny_plan_follows_store_preset():
     assert _Skinny.skinny_plan(lin, 8) == (1, 0)
     lin.fuse_silu = True
     assert _Skinny.skinny_plan(lin, 8) == (1, 0)
+
+
+def test_block_counts_and_tables():
+    """query_blocks against a loop over the tokens' blocks, and the bounded count that the
+    prefill plan decides by against the count itself, one below, at and above it."""
+    import random
+    from omniserver_amd.attention import _blocks_fit, query_blocks
+    rng = random.Random(9)
+    for _ in range(200):
+        block = rng.choice([1, 5, 16, 21, 32, 128])
+        segs = [rng.choice([1, 2, block, block + 1, int(2 ** rng.uniform(0, 11))])
+                for _ in range(rng.choice([1, 2, 7, 33]))]
+        want, off = [], 0
+        for L in segs:
+            want += [[off + s, min(block, L - s)] for s in range(0, L, block)]
+            off += L
+        table = query_blocks(segs, "cpu", block)
+        assert table.dtype == torch.int32 and table.tolist() == want
+        for most in (0, len(want) - 1, len(want), len(want) + 1, 10 ** 6):
+            assert _blocks_fit(segs, sum(segs), block, most) == (len(want) <= most)
+    assert query_blocks([], "cpu").shape == (0, 2)
