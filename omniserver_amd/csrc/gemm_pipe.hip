@@ -63,21 +63,6 @@ __device__ __forceinline__ void gp_wait_vmcnt() {
 }
 __device__ __forceinline__ void gp_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
-// h * sigmoid(1.702 h), each step rounded to fp16.  The sigmoid on the bare exp2 and reciprocal
-// instructions: with expf and an IEEE division, about 40 VALU operations a value while the
-// matrix cores wait, the vision tower's fc1 took 88.8 us at 3872 rows, now 75.5; 24.3 and
-// 22.1 at 1024.  t has 11
-// significant bits, so t times the 13-bit head of -log2(e) is exact and the exponent is
-// rounded once; the sigmoid's error before its fp16 rounding (2^-12) stays below 2^-20.
-__device__ __forceinline__ half_t gp_quick_gelu(half_t h) {
-#pragma clang fp contract(off)
-  const float t = (float)(half_t)((float)h * 1.702f);
-  constexpr float LH = -11818.0f / 8192.0f;            // head of -log2(e)
-  const float e = __builtin_amdgcn_exp2f(fmaf(t, (float)(-1.4426950408889634 - LH), t * LH));
-  const float sg = (float)(half_t)__builtin_amdgcn_rcpf(1.0f + e);
-  return (half_t)((float)h * sg);
-}
-
 // fp16 of acc + bias in the linear's order (bias_after_round: added to the fp16 rounding)
 __device__ __forceinline__ half_t gp_bias(float acc, half_t b, bool has_bias, int bar) {
 #pragma clang fp contract(off)
@@ -522,7 +507,7 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           half_t h = gp_bias(acc[i][j][q], bb[q], has_bias, a.bias_after_round);
-          if constexpr (EPI == GP_QGELU) h = gp_quick_gelu(h);
+          if constexpr (EPI == GP_QGELU) h = quick_gelu_f16(h);
           if constexpr (EPI == GP_GELU) h = gp_gelu(h);
           if constexpr (EPI == GP_RESID) h = (half_t)((float)rr[q] + (float)h);
           o[q] = h;
@@ -845,7 +830,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bigp_f16_kernel(GemmPipeArgs a) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const half_t h = gp_bias(acc[i][j][q], b[q], has_bias, a.bias_after_round);
-              o[q] = EPI == GP_QGELU ? gp_quick_gelu(h) : EPI == GP_GELU ? gp_gelu(h) : h;
+              o[q] = EPI == GP_QGELU ? quick_gelu_f16(h) : EPI == GP_GELU ? gp_gelu(h) : h;
             }
             *(half4_t*)(ob + (16 * j * a.ldo + 16 * i)) = o;
           }
@@ -1039,7 +1024,7 @@ __global__ __launch_bounds__(512, 1) void gemm_n160_kernel(GemmPipeArgs a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           half_t hv = gp_bias(acc[c][j][q], bb[q], a.bias != nullptr, a.bias_after_round);
-          if constexpr (EPI == GP_QGELU) hv = gp_quick_gelu(hv);
+          if constexpr (EPI == GP_QGELU) hv = quick_gelu_f16(hv);
           if constexpr (EPI == GP_GELU) hv = gp_gelu(hv);
           if constexpr (EPI == GP_RESID) hv = (half_t)((float)rr[q] + (float)hv);
           o[q] = hv;
@@ -1084,7 +1069,7 @@ __global__ __launch_bounds__(256) void gemm_pipe_finish_kernel(GemmPipeArgs a) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     half_t h = gp_bias(v[q], bb[q], a.bias != nullptr, a.bias_after_round);
-    if constexpr (EPI == GP_QGELU) h = gp_quick_gelu(h);
+    if constexpr (EPI == GP_QGELU) h = quick_gelu_f16(h);
     if constexpr (EPI == GP_GELU) h = gp_gelu(h);
     if constexpr (EPI == GP_RESID) h = (half_t)((float)rr[q] + (float)h);
     o[q] = h;

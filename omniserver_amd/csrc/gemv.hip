@@ -119,15 +119,6 @@ struct WStream<W_FP16> {
 };
 
 
-// x * sigmoid(1.702 x) with the three fp16 roundings of the reference's elementwise ops
-// (model/qwen2_vit.py:18-19 on fp16 tensors: 1.702 x, sigmoid, product).
-__device__ __forceinline__ half_t quick_gelu_ref(half_t h) {
-#pragma clang fp contract(off)
-  const float t = (float)(half_t)((float)h * 1.702f);
-  const float sg = (float)(half_t)(1.0f / (1.0f + expf(-t)));
-  return (half_t)((float)h * sg);
-}
-
 // Exact (erf) GELU of an fp16 value, fp32 math, one rounding (F.gelu, model/qwen2_vit.py:128).
 __device__ __forceinline__ half_t gelu_erf_ref(half_t h) {
 #pragma clang fp contract(off)
@@ -821,7 +812,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(GemvArgs a) {
           if (nt0 + c >= NT) continue;
           const int n = (nt0 + c) * 16 + c16;
           half_t h = finish_store(acc[i][c][r], a, n);
-          if constexpr (EPI == EPI_QGELU) h = quick_gelu_ref(h);
+          if constexpr (EPI == EPI_QGELU) h = quick_gelu_f16(h);
           if constexpr (EPI == EPI_GELU) h = gelu_erf_ref(h);
           if constexpr (EPI == EPI_RESID) h = (half_t)((float)a.res[(int64_t)m * a.ldr + n] + (float)h);
           a.out[(int64_t)m * a.ldo + n] = h;

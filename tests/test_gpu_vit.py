@@ -129,6 +129,33 @@ def test_gemm_epilogues(gpu, M, N, K, epi, has_bias, path, tile_rows, ksplit):
     assert (d <= tol).all(), d.max().item()
 
 
+def test_quick_gelu_every_value(gpu):
+    """QuickGELU of every finite fp16 value, through the identity product on both GEMMs: the
+    same bits from each, and x * fp16(s) for an s within 2^-20 of sigmoid(t), t = fp16(1.702 x)
+    rounded once or by way of fp32."""
+    import numpy as np
+    from omniserver_amd import vit
+    say("quick_gelu, every finite fp16 value")
+    x = np.arange(65536).astype(np.uint16).view(np.float16)
+    x = np.sort(x[np.isfinite(x)]).reshape(-1, 256)
+    got = []
+    for path in ("pipe", "tiled"):
+        lin = vit.VisionLinear(torch.eye(256, dtype=torch.float16), None, gpu, path=path)
+        out = torch.empty(x.shape, device=gpu, dtype=torch.float16)
+        lin.out(torch.from_numpy(x).to(gpu), out, vit.EPI_QGELU)
+        got.append(out.cpu().numpy())
+    assert np.array_equal(got[0].view(np.uint16), got[1].view(np.uint16))
+    x64, c = x.astype(np.float64), np.float32(1.702)
+    ok = np.zeros(x.shape, dtype=bool)
+    with np.errstate(over="ignore"):
+        for t in ((x64 * float(c)).astype(np.float16), (x.astype(np.float32) * c).astype(np.float16)):
+            s = 1 / (1 + np.exp(-t.astype(np.float64)))
+            ends = [(x64 * (s * (1 + d)).astype(np.float16)).astype(np.float16)
+                    for d in (-2.0 ** -20, 2.0 ** -20)]
+            ok |= (got[0] >= np.minimum(*ends)) & (got[0] <= np.maximum(*ends))
+    assert ok.all(), x[~ok][:10]
+
+
 @pytest.mark.parametrize("step", [64, 128])
 @pytest.mark.parametrize("segs", [[1], [31, 33], [64, 128, 65], [129, 4, 500]])
 @pytest.mark.parametrize("scale,off", [(80 ** -0.5, 0), (-0.2, 0), (80 ** -0.5, 4)])
