@@ -485,6 +485,13 @@ int omni_fp8_gemm(const void* xq, const float* sa, const void* wq, const float* 
  * mismatches[0] and the NaN ones to mismatches[1] (device memory, zeroed by the caller). */
 int omni_bf16_rne_check(unsigned long long* mismatches, void* stream);
 
+/* Self-check of the FP8 quantisers' arithmetic (no reference counterpart): adds to
+ * mismatches[0] the non-NaN fp32 bit patterns whose hardware e4m3fn conversion differs from
+ * the rounding written out in integers, to mismatches[1] and [2] the quotients by a scale that
+ * differ from fp32 division, for 11-bit numerators (fp16, bf16: every pair of significands)
+ * and for 24-bit ones (2^31 pairs) (device memory, three counts, zeroed by the caller). */
+int omni_fp8_codes_check(unsigned long long* mismatches, void* stream);
+
 /* The kernel omni_fp8_gemm runs for a shape (no reference counterpart: it tells a caller
  * or a test which form covers the shape): 0 one 128 x 128 tile per workgroup (K < 512),
  * 1 the pipelined persistent 256 x 128 tiles, 2 the persistent 256 x 256 tiles (where whole

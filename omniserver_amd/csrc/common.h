@@ -99,12 +99,14 @@ __host__ __device__ __forceinline__ float e4m3fn_to_f32(uint8_t v) {
 // e4m3 quantisation by a common scale, q = e4m3(v / s), eight values at a time.  What it must
 // equal is the correctly rounded fp32 division followed by f32_to_e4m3fn; done that way it is
 // about 35 VALU operations a value and the quantisers ran at a fifth of the memory rate.
-// Instead v / s is v * (1/s) corrected by its own fma residual, with the reciprocal (correctly
-// rounded, once per scale): one correction reproduces the division for numerators of at most
-// 11 significant bits (fp16, bf16), two for any (the residual is exact in fma arithmetic and
-// the corrected quotient rounds as the division does, save for a divisor whose significand
-// is all ones).  The codes come from gfx950's v_cvt_pk_fp8_f32, which equals f32_to_e4m3fn on
-// every fp32 value that is not NaN (all 2^32 checked; it gives 0xff for either NaN sign).  A
+// Instead v / s is Markstein's fma-corrected quotient (IBM J. Res. Dev. 34, 1990): v * (1/s)
+// corrected by its own fma residual, with the reciprocal (correctly rounded, once per scale).
+// One correction reproduces the division for numerators of at most 11 significant bits (fp16,
+// bf16: every pair of significands is compared by omni_fp8_codes_check), two for any (the
+// residual is exact in fma arithmetic and the corrected quotient rounds as the division does,
+// save for a divisor whose significand is all ones; 2^31 pairs compared there).  The codes come
+// from gfx950's v_cvt_pk_fp8_f32, which equals f32_to_e4m3fn on every fp32 value that is not NaN
+// (all compared there; it gives 0xff for either NaN sign).  A
 // scale outside [2^-60, 2^60] or with an all-ones significand, or a chunk with a NaN quotient,
 // takes the long way.
 struct Fp8Scale {

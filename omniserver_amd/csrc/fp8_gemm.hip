@@ -1477,3 +1477,48 @@ extern "C" int omni_bf16_rne_check(unsigned long long* mismatches, void* stream)
   OMNI_CHECK_LAUNCH();
   return OMNI_OK;
 }
+
+// Device check of the quantisers' arithmetic (fp8_codes8) against what it must equal:
+// mismatches[0] counts the non-NaN fp32 bit patterns whose hardware e4m3 conversion is not
+// f32_to_e4m3fn's, mismatches[1] the quotients of 11-bit numerators (every pair of significands)
+// and mismatches[2] those of 24-bit numerators (256 per divisor significand) whose corrected
+// product is not the fp32 division.  Significands decide: within the plain scales' exponents
+// nothing that reaches a code above 0 over- or underflows.
+__global__ __launch_bounds__(256) void fp8_codes_check_kernel(unsigned long long* mismatches) {
+#pragma clang fp contract(off)
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;      // 2^23 threads
+  uint32_t bad[3] = {0, 0, 0};
+  for (uint32_t k = 0; k < 512; k += 2) {
+    const uint32_t u0 = (i << 9) | k, u1 = u0 | 1u;
+    const float v0 = __builtin_bit_cast(float, u0), v1 = __builtin_bit_cast(float, u1);
+    if (__builtin_isunordered(v0, v1)) continue;          // exponents: both NaN or the first inf
+    const uint32_t c = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v0, v1, 0, false);
+    bad[0] += (c & 0xffu) != f32_to_e4m3fn(v0);
+    bad[0] += ((c >> 8) & 0xffu) != f32_to_e4m3fn(v1);
+  }
+  if ((i & 0x3fffffu) == 0x3fc000u) {                      // +-inf, whose odd neighbour is a NaN
+    const float v = __builtin_bit_cast(float, i << 9);
+    bad[0] += ((uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v, v, 0, false) & 0xffu) != f32_to_e4m3fn(v);
+  }
+  const Fp8Scale d(__builtin_bit_cast(float, 0x3f800000u | i));
+  if (d.plain) {
+    for (uint32_t n = 1024; n < 2048; ++n)
+      bad[1] += fp8_quotient<1>((float)n, d) != (float)n / d.s;
+    uint32_t h = i * 2654435761u;
+    for (uint32_t n = 0; n < 256; ++n) {
+      h = h * 1664525u + 1013904223u;
+      const float v = __builtin_bit_cast(float, 0x3f800000u | (h >> 9));
+      bad[2] += fp8_quotient<2>(v, d) != v / d.s;
+    }
+  }
+  for (int k = 0; k < 3; ++k)
+    if (bad[k]) atomicAdd(&mismatches[k], (unsigned long long)bad[k]);
+}
+
+extern "C" int omni_fp8_codes_check(unsigned long long* mismatches, void* stream) {
+  if (!mismatches || ((uintptr_t)mismatches & 7)) return OMNI_EINVAL;
+  hipLaunchKernelGGL(fp8_codes_check_kernel, dim3(1u << 15), dim3(256), 0, (hipStream_t)stream,
+                     mismatches);
+  OMNI_CHECK_LAUNCH();
+  return OMNI_OK;
+}

@@ -152,6 +152,18 @@ def test_bf16_rounding_exhaustive(gpu):
     assert mism.tolist() == [0, 0]
 
 
+def test_fp8_codes_exhaustive(gpu):
+    """The quantisers' hardware e4m3 conversion against the integer rounding on every fp32 value
+    that is not NaN, and their corrected quotients against fp32 division: every pair of
+    significands for 11-bit numerators, 2^31 pairs for 24-bit ones."""
+    from omniserver_amd._lib import call, ptr, stream
+    say("e4m3 conversion on all fp32 inputs, quotients on all significand pairs")
+    mism = torch.zeros(3, dtype=torch.int64, device=gpu)
+    call("omni_fp8_codes_check", ptr(mism), stream())
+    torch.cuda.synchronize()
+    assert mism.tolist() == [0, 0, 0]
+
+
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("M,K,N", [(1, 512, 128), (16, 640, 2048), (17, 8960, 1536),
                                    (64, 8960, 1536), (65, 1536, 2048), (130, 8960, 1536),
