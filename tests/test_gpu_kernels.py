@@ -427,20 +427,27 @@ def test_w4a16_gemm(gpu, M, K, N, bias, silu):
                 assert d <= 1e-3 * max(1.0, e32.abs().max().item()), (ks, pr, d)
 
 
+# form: slices of (int4, fp16) with K split, 4 the 16-column workgroups, 2 the 64-column ones
 @pytest.mark.parametrize("fmt", ["int4", "fp16"])
-@pytest.mark.parametrize("M,K,N,bias", [(1, 8960, 1536, False), (33, 8960, 1536, True),
-                                        (16, 8960, 1536, True), (64, 1536, 2048, True),
-                                        (49, 1536, 272, True), (64, 3584, 272, True),
-                                        (17, 3200, 80, True), (64, 640, 128, False),
-                                        (64, 1536, 4608, True), (3, 512, 16, True)])
-def test_skinny_finished_split(gpu, fmt, M, K, N, bias):
+@pytest.mark.parametrize("M,K,N,bias,form", [
+    (1, 8960, 1536, False, 4), (33, 8960, 1536, True, (10, 20)), (16, 8960, 1536, True, 4),
+    (17, 8960, 1536, False, (10, 20)), (64, 1536, 2048, True, 4), (49, 1536, 272, True, 4),
+    (64, 3584, 272, True, (6, 8)), (17, 3200, 80, True, 4), (64, 640, 128, False, 4),
+    (64, 1536, 4608, True, (6, 6)), (3, 512, 16, True, 4), (48, 1536, 4608, True, 2),
+    (16, 4992, 4608, False, (6, 11)), (64, 384, 128, True, 2)])
+def test_skinny_finished_split(gpu, fmt, M, K, N, bias, form, monkeypatch):
     """The finished linear at up to 64 rows on each of its forms (16 columns a workgroup, K
-    slices and a finish launch, 64 columns) and at the edges of their rule: within the other linears' tolerance of the fp32 oracle, bias
-    rounded as the format's store epilogue rounds it, nothing written past the output's
-    columns; an output the finish cannot store to (rows 2 halfs apart from 8 bytes) takes the
-    store kernel."""
+    slices and a finish launch, 64 columns; the form is asserted, and that the finish runs
+    exactly with the slices) and at the edges of their rule: within the other linears'
+    tolerance of the fp32 oracle, bias rounded as the format's store epilogue rounds it, nothing
+    written past the output's columns; an output the finish cannot store to (rows 2 halfs apart
+    from 8 bytes) takes the store kernel."""
+    from omniserver_amd import linear
     from omniserver_amd.linear import F16Linear, GPTQLinear
-    say(f"skinny finished split {fmt} M={M} K={K} N={N} bias={bias}")
+    say(f"skinny finished split {fmt} M={M} K={K} N={N} bias={bias} form={form}")
+    called = []
+    own = linear.call
+    monkeypatch.setattr(linear, "call", lambda name, *a: (called.append(name), own(name, *a))[1])
     b = f16((N,), 75, 0.5) if bias else None
     if fmt == "int4":
         qw, sc = _gptq(K, N, 76 + K + N)
@@ -451,9 +458,14 @@ def test_skinny_finished_split(gpu, fmt, M, K, N, bias):
     x = f16((M, K), 78)
     e = ref.linear(x.float(), W, None if b is None else b.float(), bias_after_round=fmt == "int4")
     tol = 2e-3 * max(1.0, e.abs().max().item())
+    split = isinstance(form, tuple)
+    ks, preset = lin.skinny_plan(M)
+    assert (ks if split else (ks, preset)) == (form[fmt == "fp16"] if split else (1, form))
     for pad in (8, 2):
         buf = torch.full((M, N + pad), 7.0, device=gpu, dtype=torch.float16)
+        called.clear()
         lin.forward_out(x.to(gpu), buf[:, :N])
+        assert ("omni_gemm_finish" in called) == (split and pad == 8)
         got = buf.cpu()
         assert (got[:, :N].float() - e).abs().max().item() <= tol
         assert (got[:, N:] == 7.0).all()
@@ -1414,9 +1426,9 @@ def test_fp8_gemm_big_tiles_ragged_rows(gpu, M, N, K, bias):
                                    (1937, 17920, 1536)])
 def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
     """The gate|up product with the SiLU-mul in its epilogue: every output form bit-equal to
-    the product followed by silu_mul, more and fewer tiles than CUs, a last row
-    tile that repeats rows, the partial maxima's maximum the output's, columns past the output untouched; shapes off
-    the 256 x 256 tiles are refused."""
+    the product followed by silu_mul, more and fewer tiles than CUs, a last row tile that
+    repeats rows, the partial maxima's maximum the output's, columns past the output untouched;
+    shapes off the 256 x 256 tiles have no grid and are refused."""
     from omniserver_amd import fused_ops as F
     from omniserver_amd._lib import call, lib, ptr, stream
     from omniserver_amd.linear import FP8Linear
@@ -1425,6 +1437,8 @@ def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
     xq, sa = lin.quantize_input(f16((M, K), 167).to(gpu))
     grid = lib().omni_fp8_gemm_silu_grid(M, N, K)
     assert grid > 0 and lib().omni_fp8_gemm_silu_grid(255, N, K) == 0
+    assert lib().omni_fp8_gemm_silu(ptr(xq), ptr(sa), ptr(lin.weight_fp8), ptr(lin.weight_scale),
+                                    ptr(xq), N // 2, None, 255, N, K, lin.OUT_BF16, stream()) == -2
     for mode in (lin.OUT_F16_VIA_BF16, lin.OUT_BF16, lin.OUT_F16):
         dt = torch.bfloat16 if mode == lin.OUT_BF16 else torch.float16
         want = F.silu_mul(lin.gemm_out(xq, sa, torch.empty(M, N, device=gpu, dtype=dt), mode))
@@ -1439,25 +1453,37 @@ def test_fp8_gemm_silu_equals_two_launches(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("rowwise", [False, True])
-@pytest.mark.parametrize("M", [1, 255, 256, 300, 1000, 1025])
-def test_fp8_mlp_fused_silu(gpu, M, rowwise):
-    """The FP8 MLP on both sides of the fused gate|up rule: bit-equal to its linears called one
-    by one with silu_mul between them, also where a forward hook keeps it off the fused form."""
+@pytest.mark.parametrize("M", [1, 255, 256, 257, 300, 1000, 1025])
+def test_fp8_mlp_fused_silu(gpu, M, rowwise, monkeypatch):
+    """The FP8 MLP on both sides of the fused gate|up rule (which side is asserted, and that the
+    fused product ran): bit-equal to its linears called one by one with silu_mul between them,
+    also where a forward hook keeps it off the fused form."""
     from omniserver_amd import fused_ops as F
+    from omniserver_amd import linear
     from omniserver_amd.linear import FP8Linear
     from omniserver_amd.qwen2_llm import MLP
-    say(f"fp8 mlp fused silu M={M} rowwise={rowwise}")
+    from omniserver_amd._lib import lib
+    fused = M > 256        # up to 256 rows the two launches are one round of smaller tiles
+    say(f"fp8 mlp fused silu M={M} rowwise={rowwise} fused={fused}")
+    called = []
+    own = linear.call
+    monkeypatch.setattr(linear, "call", lambda name, *a: (called.append(name), own(name, *a))[1])
     gu = FP8Linear(f16((17920, 1536), 171, 0.05).to(gpu), rowwise=rowwise)
     down = FP8Linear(f16((1536, 8960), 172, 0.05).to(gpu), rowwise=rowwise)
     x = f16((M, 1536), 173).to(gpu)
     mlp = MLP(gu, down)
+    assert (lib().omni_fp8_gemm_silu_grid(M, gu.N, gu.K) > 0) == fused
     want = down(F.silu_mul(gu(x)))
+    called.clear()
     assert torch.equal(mlp(x), want)
+    assert ("omni_fp8_gemm_silu" in called) == fused and called.count("omni_fp8_gemm") == 2 - fused
     seen = []
     gu.register_forward_hook(lambda m, args, out: seen.append(out.shape))
     down.register_forward_pre_hook(lambda m, args: seen.append(len(args)))
+    called.clear()
     assert torch.equal(mlp(x), want)
     assert seen == [(M, 17920), 1]
+    assert "omni_fp8_gemm_silu" not in called
 
 
 @pytest.mark.parametrize("prequant", [False, True])
@@ -1664,17 +1690,17 @@ def test_fp8_prequant_chain(gpu):
     assert (d <= tol + 1e-6).all(), (d - tol).max().item()
 
 
-@pytest.mark.parametrize("M,N,K,epi", [(4000, 3840, 256, 0), (3872, 5120, 256, 4), (300, 33024, 256, 0),
-                                       (4095, 5120, 384, 5), (2047, 17920, 256, 1)])
-@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K,epi,bias", [
+    (4000, 3840, 256, 0, False), (300, 33024, 256, 0, False), (2047, 17920, 256, 1, False),
+    (3872, 5120, 256, 4, False), (3872, 5120, 256, 4, True), (4095, 5120, 384, 5, False),
+    (4095, 5120, 384, 5, True)])
 def test_f16_big_tiles_ragged_rows(gpu, M, N, K, epi, bias):
     """The persistent 256-row tiles at row counts off a multiple of 256 (the last row tile
-    repeats up to 255 rows of the one before it) in every epilogue they have (0 STORE, 1 SILU,
-    4 QGELU, 5 GELU; biases staged per tile; tail columns): bit-equal to the 128 x 128 tiles, and nothing written past the rows or the columns."""
+    repeats up to 255 rows of the one before it) in every epilogue they have (0 STORE and 1 SILU
+    without a bias, 4 QGELU and 5 GELU with and without one, staged per tile; tail columns):
+    bit-equal to the 128 x 128 tiles, and nothing written past the rows or the columns."""
     import ctypes
     from omniserver_amd._lib import call, lib, ptr, stream
-    if bias and epi in (0, 1):
-        pytest.skip("no bias in this form")
     r, c, k = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     lib().omni_packed_gemm_pipe_plan(M, N, K, 1, epi, int(bias), 0, 0, ctypes.byref(r),
                                      ctypes.byref(c), ctypes.byref(k))
