@@ -524,10 +524,10 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
   gp_wait_vmcnt<0>();                  // drain the clamped tail loads before exit
 }
 
-// Persistent 256 x 256 or 256 x 192 (PARTIAL) tiles for the packed fp16 weights (STORE
-// without a bias, QGELU, GELU, SILU and PARTIAL, M >= 256, N a multiple of the tile width; rows past the last multiple of
-// 256 take a tile that ends at row M - 1 and repeats rows of the tile before it: the same
-// bytes written twice, no bound on loads or stores):
+// Persistent 256 x 256 or 256 x 192 (PARTIAL) tiles for the packed fp16 weights (unbiased STORE,
+// QGELU, GELU, SILU and PARTIAL; M >= 256, N a multiple of the tile width).  Rows past the last
+// multiple of 256 take a tile that ends at row M - 1 and repeats rows of the tile before it:
+// the same bytes written twice, no bound on loads or stores.
 // 8 waves (two per SIMD: 2 along m x 4 along n), each owning a 128 (m) x 16 NIW (n) block,
 // so every operand byte staged through LDS feeds twice the MFMA work it feeds in the
 // 256 x 128 tiles above; two stages of 32 KB of x and 8 NIW KB of w (x rows XOR-swizzled as
@@ -540,16 +540,15 @@ __global__ __launch_bounds__(128 * WM, 1) void gemm_pipe_kernel(GemmPipeArgs a) 
 // leave CUs idle), read and stored by the same code for NIW / 2 column tiles per wave.
 // PARTIAL writes each K slice's fp32 sums to part[slice][M][N] for the consumer to add in
 // slice order (config 5's down projection at M = 4096: 128 tiles of 256 x 192 in two
-// slices fill the 256 CUs once).  A
-// tile's biases ride with its first stage into an LDS slot of their own (two, by tile parity):
-// read from global memory in the epilogue they would wait for the next tile's stages.  The
-// vision tower's linears, 256 x 128 tiles / this, us: 1280 -> 5120 + QGELU at 3872 rows 76.9 /
-// 75.5, 2100 52.4 / 46.5, 2852 54 / 49.5;
-// 5120 -> 5120 + GELU at 2100 165 / 141.6.  Same k order per output as the
-// kernel above within a slice: one-slice results equal its bit for bit.  MI355X, us
-// (256 x 128 or 128 x 192 / this, interleaved, median of 7): M = 4096 gate_up + SiLU
+// slices fill the 256 CUs once).  A tile's biases ride with its first stage into an LDS slot
+// of their own (two, by tile parity): read from global memory in the epilogue they would wait
+// for the next tile's stages.  Same k order per output as the kernel above within a slice:
+// one-slice results equal its bit for bit.
+// MI355X, us (256 x 128 or 128 x 192 / this, interleaved, median of 7): M = 4096 gate_up + SiLU
 // 240.1 / 222.6; M = 8192 gate_up 469.7 / 397.5, down 238.6 / 200.2 (four waves of 128 x 128:
-// 440.0 and 216.5).
+// 440.0 and 216.5).  The vision tower's linears: 1280 -> 5120 + QGELU at 3872 rows 76.9 / 75.5,
+// 2100 52.4 / 46.5, 2852 54 / 49.5; 5120 -> 5120 + GELU at 2100 165 / 141.6.
+
 // The wave's lane index computed afresh (v_mbcnt in an asm block, which the compiler can
 // neither hoist nor merge with an earlier value): for addresses needed once per tile, so
 // that neither they nor the lane index stay live beside 256 accumulators.
@@ -1253,9 +1252,10 @@ extern "C" int omni_f16_gemm_pipe(const void* x, int ldx, const void* w, const v
 
 // omni_packed_gemm_pipe's tiling for a shape: tile rows and columns and K slices, from the
 // caller's tile_rows / ksplit (0: chosen).  128 x 192 and persistent 256 x 256 tiles only
-// where both were chosen; the 256 x 256 ones (fp16 weights, unbiased STORE, QGELU, GELU, SILU, M
-// from 256, N a multiple of 256) where rounds of the grid times the tile's cost (per 128 x 128
-// outputs: GP_BIG_COST, against 1 or GP_WIDE_COST) come out below the other plan's.
+// where both were chosen; the 256 x 256 ones (fp16 weights; unbiased STORE, QGELU, GELU and
+// SILU at M from 256 and N a multiple of 256) where rounds of the grid times the tile's cost
+// (per 128 x 128 outputs: GP_BIG_COST, against 1 or GP_WIDE_COST) come out below the other
+// plan's.
 static void gp_packed_plan(int M, int N, int K, int fmt, int epilogue, bool has_bias, int tile_rows,
                            int ksplit, int& rows, int& cols, int& ks) {
   rows = tile_rows ? tile_rows : gp_tile_rows(M, N);
@@ -1323,11 +1323,20 @@ static void gp_packed_plan(int M, int N, int K, int fmt, int epilogue, bool has_
     const double cur = rounds((int64_t)ceil_div(M, rows) * (N / cols)) * (rows * cols) / 16384.0 *
                        (cols == 192 ? GP_WIDE_COST : 1.0);
     // a half-tile tail round (gp_big_tail_cols) measured at 0.65 of a whole one: M = 4096
-    // gate_up + SiLU 204.9 against 221.1 us with whole tiles only
+    // gate_up + SiLU 204.9 against 221.1 us with whole tiles only.  Off the multiples of 256,
+    // where the repeated rows are work too, 0.75 after a single round of plain or SiLU tiles and
+    // 4 % ahead in all: without that the estimate chose tiles that measured behind (us, 256 x 128
+    // or 128 x 192 / 256 x 256): 1536 -> 17920 + SiLU at 2561 .. 2746 rows 160 / 166; 3584 ->
+    // 37888 + SiLU at 257 158 / 165, 511 162 / 164; 3584 -> 4608 at 4056 152 / 158.  (QuickGELU
+    // and GELU after one round: 5120 -> 5120 + GELU at 3925 ahead by 3 %.)
+    const bool ragged = M % 256 != 0;
     const int64_t tb = (int64_t)ceil_div(M, 256) * (N / 256);
-    const double big = (gp_big_tail_cols(M, N) < N ? (double)(tb / cus) + GP_TAIL_COST : rounds(tb)) *
+    const bool slow_tail = ragged && tb / cus == 1 && K >= 1024 &&
+                           (epilogue == GP_STORE || epilogue == GP_SILU);
+    const double tail = slow_tail ? 0.75 : GP_TAIL_COST;
+    const double big = (gp_big_tail_cols(M, N) < N ? (double)(tb / cus) + tail : rounds(tb)) *
                        4.0 * GP_BIG_COST;
-    if (big < cur) {
+    if (big < (ragged ? 0.96 : 1.0) * cur) {
       rows = 256;
       cols = 256;
     }

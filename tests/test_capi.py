@@ -236,3 +236,30 @@ def test_packed_silu160_plan(so):
     assert plan(1024, 3840, 1280, 1, 0)[1] != 160          # 192 against 240
     assert plan(1024, 5120, 1280, 1, 2)[1] != 160          # partial sums keep their plan
     assert plan(4096, 5120, 1280, 1, 4)[1] != 160          # more than one round
+
+
+def test_packed_big_tiles_plan(so):
+    """Off the multiples of 256 rows the persistent 256 x 256 tiles run where they are clearly
+    ahead of the smaller tiles: not with only a nearly empty last round less, nor for one round
+    and a tail of plain or SiLU tiles; multiples of 256 and the GELU forms keep the plain
+    estimate."""
+    import ctypes
+    from omniserver_amd._lib import lib
+    L = lib()
+
+    def plan(M, N, K, epi, bias=0):
+        r, c, k = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+        assert L.omni_packed_gemm_pipe_plan(M, N, K, 1, epi, bias, 0, 0, ctypes.byref(r),
+                                            ctypes.byref(c), ctypes.byref(k)) == 0
+        return r.value, c.value, k.value
+
+    big = (256, 256, 1)
+    # 17920 columns: 4 rounds against 7 of 256 x 128 (2561 .. 2816 rows), 3 and a tail (2817 ..)
+    assert plan(2561, 17920, 1536, 1) == plan(2815, 17920, 1536, 1) == (256, 128, 1)
+    assert plan(2816, 17920, 1536, 1) == big and plan(2817, 17920, 1536, 1) == big
+    # one round and a tail: SiLU and plain tiles at ragged rows only off it
+    assert plan(511, 37888, 3584, 1) == (256, 128, 1) and plan(512, 37888, 3584, 1) == big
+    assert plan(4095, 4608, 3584, 0) == (128, 192, 1) and plan(4096, 4608, 3584, 0) == big
+    assert plan(3872, 5120, 1280, 4, 1) == big and plan(3925, 5120, 5120, 5, 1) == big
+    # one round of them against two: ragged rows too
+    assert plan(650, 17920, 1536, 1) == big and plan(2877, 4608, 3584, 0) == big
