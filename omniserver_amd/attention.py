@@ -95,10 +95,16 @@ def prefill_plan(seg_lengths, starts, nh: int, nkv: int, cus: int) -> tuple:
     keys = max(map(operator.add, starts, seg_lengths), default=0)
     items_fit = lambda most: _blocks_fit(seg_lengths, tokens, QBLOCK, most // nh)
     wgs_fit = lambda rows, most: _blocks_fit(seg_lengths, tokens, rows // group, most // nkv)
-    # A few short contexts: the split kernel starts and merges in 2-3 us less (1 x 256: 6.5
-    # against 7.5 us, 16 x 24: 4.5 against 6.5) until its items queue (2 x 256: 9.0 against
-    # 7.6) or the keys are many (a 128-token chunk at 500 keys: level).
-    if keys <= 320 and items_fit(cus if keys > 64 else 2 * cus):
+    # Short contexts: the split kernel starts and merges in 1-2.5 us less until its items queue
+    # or its four waves' key steps add up, sooner for blocks of few rows, of which the rows
+    # kernel wastes less.  Us, split / rows, 12 / 2 heads: 16 tokens at 64 keys 4.2 / 6.3, 320
+    # 7.2 / 8.4, 600 9.4 / 9.9, 800 11.6 / 11.5; one token at 64 4.5 / 5.2, 256 6.3 / 6.0, 420
+    # 8.4 / 7.6; 256 tokens at 600 9.8 / 10.2; without grouping (16 / 16) 128 at 420 8.5 / 9.3,
+    # 600 11.4 / 10.5.  Two rounds of items: 8 x 64 4.8 / 6.6, 4 x 128 6.3 / 6.9, 4 x 128 at 320
+    # 10.4 / 8.7; 32 single tokens at 64 4.8 / 5.3, 80 6.0 / 5.6.  Three: 8 x 100 8.9 / 7.2.
+    full = max(seg_lengths, default=0) * group >= 32
+    if ((keys <= (320 if not full else 640 if group > 1 else 448) and items_fit(cus))
+            or (keys <= (128 if full else 64) and items_fit(2 * cus))):
         return ("omni_prefill_attention_split", QBLOCK, ())
     # Rows to spare for every CU only in 128s: fewer rows per workgroup while those still fit
     # one round of the CUs, with the keys dealt to as many groups as the waves allow.  A long

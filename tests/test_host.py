@@ -494,3 +494,19 @@ def test_block_counts_and_tables():
         for most in (0, len(want) - 1, len(want), len(want) + 1, 10 ** 6):
             assert _blocks_fit(segs, sum(segs), block, most) == (len(want) <= most)
     assert query_blocks([], "cpu").shape == (0, 2)
+
+
+def test_prefill_plan_short_contexts():
+    """The split kernel's range at its edges: one round of its (block, head) items up to 640
+    keys (448 without head grouping, 320 where no block fills a 32-row tile), two rounds up to
+    128 (64); the row-tile kernel beyond."""
+    from omniserver_amd.attention import prefill_plan
+    split = lambda segs, starts, nh, nkv: prefill_plan(segs, starts, nh, nkv, 256)[0].endswith("split")
+    assert split([16], [624], 12, 2) and not split([16], [625], 12, 2)
+    assert split([5], [315], 12, 2) and not split([5], [316], 12, 2)       # 30 rows
+    assert split([6], [634], 12, 2) and not split([6], [635], 12, 2)       # 36 rows
+    assert split([40], [408], 16, 16) and not split([40], [409], 16, 16)
+    assert split([128] * 4, [0] * 4, 12, 2) and not split([129] * 3, [0] * 3, 12, 2)
+    assert split([1] * 32, [63] * 32, 12, 2) and not split([1] * 32, [64] * 32, 12, 2)
+    assert split([336], [0], 12, 2) and not split([337], [0], 12, 2)       # 252 and 264 items
+    assert not split([64] * 11, [0] * 11, 12, 2)                           # 528 items
