@@ -189,7 +189,9 @@ int omni_prefill_attention_split(const void* q, int q_stride, const void* k_cach
 /* The same attention with query blocks of up to 32 tokens (qblocks counts <= 32): one
  * workgroup per (block, KV head) loads each 32-key K/V tile once into LDS for all the
  * group's query heads (n_heads / n_kv_heads <= 8); outputs equal omni_prefill_attention's
- * bit for bit.  For long segments. */
+ * bit for bit.  omni_prefill_attention_rows is faster wherever the two were measured, and what this
+ * library's own prefills take; this entry point and its two-group form stay for callers that
+ * bind this header and rely on those bits. */
 int omni_prefill_attention_gqa(const void* q, int q_stride, const void* k_cache,
                                const void* v_cache, int pool_rows, int max_len,
                                const int64_t* slots, const int64_t* kv_len, const int* qblocks,

@@ -38,7 +38,8 @@ from ._lib import call, ptr, stream
 from .hostio import to_device
 
 QBLOCK = 16
-QBLOCK_GQA = 32          # blocks of the shared-tile kernels
+# blocks of the shared-tile entry points, kept for callers of the C header alone
+QBLOCK_GQA = 32
 # the rows kernel's most query heads per KV head
 ROWS_MAX_GROUP = 32
 # (block, head) items per CU up to which the split kernel, not the per-wave one, runs
