@@ -225,6 +225,12 @@ int omni_prefill_attention_rows(const void* q, int q_stride, const void* k_cache
                                 int head_dim, float scale, int rows, int groups,
                                 void* stream);
 
+/* The qblocks table of a packed batch, on the host: for segments of seg_lengths[nseg] >= 0
+ * tokens in order, (first token, count) of every block of at most block tokens into
+ * table[capacity][2].  Returns the number of blocks (at most the tokens / block + nseg), -1 for
+ * a negative length, block < 1 or more than capacity. */
+int omni_query_blocks(const int* seg_lengths, int nseg, int block, int* table, int capacity);
+
 /* ---------------------------------------------------------------- linears */
 
 /* Epilogues of the skinny GEMMs. */

@@ -67,6 +67,7 @@ SIGNATURES = {
                                           _I, _I, _F, _P],
     "omni_prefill_attention": [_P, _I, _P, _P, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _F,
                                _P],
+    "omni_query_blocks": [_P, _I, _I, _P, _I],
     "omni_prefill_attention_rows": [_P, _I, _P, _P, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I,
                                     _F, _I, _I, _P],
     "omni_prefill_attention_split": [_P, _I, _P, _P, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I,

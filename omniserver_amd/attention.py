@@ -34,8 +34,7 @@ from array import array
 
 import torch
 
-from ._lib import call, ptr, stream
-from .hostio import to_device
+from ._lib import call, lib, ptr, stream
 
 QBLOCK = 16
 # blocks of the shared-tile entry points, kept for callers of the C header alone
@@ -56,23 +55,17 @@ def num_cus(device) -> int:
 
 
 def query_blocks(seg_lengths, device, block: int = QBLOCK) -> torch.Tensor:
-    """int32 [nqb, 2] (first token, count) covering every segment in blocks of <= block.  Built
-    a segment at a time: on a new ragged batch it is part of the first layer's call."""
-    first, count = [], []
-    off = 0
-    for L in seg_lengths:
-        first += range(off, off + L, block)
-        whole, rest = divmod(L, block)
-        count += [block] * whole
-        if rest:
-            count.append(rest)
-        off += L
-    table = [0] * (2 * len(first))
-    table[::2], table[1::2] = first, count
-    if not table:
-        return torch.empty(0, 2, dtype=torch.int32, device=device)
-    return to_device(torch.frombuffer(array("i", table), dtype=torch.int32), torch.int32,
-                     device).view(-1, 2)
+    """int32 [nqb, 2] (first token, count) covering every segment in blocks of <= block.  On a
+    new batch this is part of the first layer's call, so the table is filled natively, straight
+    into the staging buffer."""
+    device = torch.device(device)
+    most = sum(seg_lengths) // block + len(seg_lengths)
+    host = torch.empty(most, 2, dtype=torch.int32, pin_memory=device.type == "cuda")
+    lens = array("i", seg_lengths)
+    n = lib().omni_query_blocks(lens.buffer_info()[0], len(lens), block, host.data_ptr(), most)
+    if n < 0:
+        raise ValueError(f"segments {list(seg_lengths)} in blocks of {block}")
+    return host[:n].to(device, non_blocking=True)
 
 
 def _blocks_fit(seg_lengths, tokens: int, block: int, most: int) -> bool:

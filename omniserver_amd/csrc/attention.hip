@@ -1272,6 +1272,28 @@ static int prefill_args(PrefillArgs& a, const void* q, int q_stride, const void*
   return OMNI_OK;
 }
 
+// The host table of query blocks the prefill entry points take: every segment in blocks of at
+// most block tokens.  Returns their number, or OMNI_EINVAL.
+extern "C" int omni_query_blocks(const int* seg_lengths, int nseg, int block, int* table,
+                                 int capacity) {
+  if (nseg < 0 || block < 1 || capacity < 0 || (nseg > 0 && !seg_lengths)) return OMNI_EINVAL;
+  if (capacity > 0 && !table) return OMNI_EINVAL;
+  int n = 0;
+  int64_t first = 0;
+  for (int s = 0; s < nseg; ++s) {
+    const int len = seg_lengths[s];
+    if (len < 0 || first + len > 0x7fffffff) return OMNI_EINVAL;
+    for (int64_t o = 0; o < len; o += block) {
+      if (n == capacity) return OMNI_EINVAL;
+      table[2 * n] = (int)(first + o);
+      table[2 * n + 1] = (int)(len - o < block ? len - o : block);
+      ++n;
+    }
+    first += len;
+  }
+  return n;
+}
+
 // Causal varlen attention for packed query tokens over the pool.
 //   qblocks int32 [nqb][2]: (first token, count <= 16); the tokens of a block share
 //   slots[t] and have increasing kv_len.  out fp16 rows of out_stride elements.

@@ -494,6 +494,9 @@ def test_block_counts_and_tables():
         for most in (0, len(want) - 1, len(want), len(want) + 1, 10 ** 6):
             assert _blocks_fit(segs, sum(segs), block, most) == (len(want) <= most)
     assert query_blocks([], "cpu").shape == (0, 2)
+    assert query_blocks([3, 0, 2], "cpu", 2).tolist() == [[0, 2], [2, 1], [3, 2]]
+    with pytest.raises(ValueError):
+        query_blocks([5, -1], "cpu", 2)
 
 
 def test_prefill_plan_short_contexts():
