@@ -192,17 +192,17 @@ class _Skinny(nn.Module):
         along K as tile_ksplit says unless ``ksplit`` is given)."""
         epi = EPI_SILU if self.fuse_silu else EPI_STORE
         M = x2d.shape[0]
-        if 0 < M <= MAX_SKINNY_M and not self.fuse_silu and preset is None and ksplit is None:
-            ks, pr = _skinny_plan(self.fmt, self.K, self.N, M)
-            if ks == 1:
-                preset = pr
-            elif not ((out.data_ptr() & 7) or (out.stride(0) & 3)):
+        if 0 < M <= MAX_SKINNY_M and preset is None and ksplit is None:
+            ks, pr = (1, None) if self.fuse_silu else _skinny_plan(self.fmt, self.K, self.N, M)
+            if ks > 1 and not ((out.data_ptr() & 7) or (out.stride(0) & 3)):
                 ws = torch.empty(self.partial_slices(ks) * M * self.N, device=x2d.device,
                                  dtype=torch.float32)
                 S = self.forward_partial(x2d, ws, ks, pr)
                 call("omni_gemm_finish", ptr(ws), S, ptr(self.bias), int(self.fmt == "int4"),
                      ptr(out), out.stride(0), M, self.N, stream())
                 return out
+            self._call(x2d, out, None, epi, 1, self.store_preset if ks > 1 or pr is None else pr)
+            return out
         ks = self.tile_ksplit(M) if ksplit is None else ksplit
         if M > MAX_SKINNY_M and epi == EPI_STORE and ks > 1:
             ws = torch.empty(self.partial_slices(ks) * M * self.N, device=x2d.device,
