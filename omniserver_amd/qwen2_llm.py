@@ -83,30 +83,30 @@ class Attention(nn.Module):
         self.o_proj = o_proj
 
 
-_ALL_HOOKS = tuple(getattr(_module, f"_global_{k}_hooks", ())
-                   for k in ("forward", "forward_pre", "backward", "backward_pre"))
+_ALL_FORWARD, _ALL_FORWARD_PRE, _ALL_BACKWARD, _ALL_BACKWARD_PRE = (
+    getattr(_module, f"_global_{k}_hooks", ())
+    for k in ("forward", "forward_pre", "backward", "backward_pre"))
 _MODULE_CALL = nn.Module.__call__
-_FP8_METHODS = tuple((n, vars(FP8Linear)[n])
-                     for n in ("forward", "forward_prequant", "quantize_input", "gemm_out"))
+_FORWARD, _PREQUANT = FP8Linear.forward, FP8Linear.forward_prequant
+_QUANTIZE, _GEMM = FP8Linear.quantize_input, FP8Linear.gemm_out
 
 
 def _fp8_as_built(mod) -> bool:
     """Whether mod is an FP8Linear whose calls nothing watches or replaces: no subclass, no
-    method set on it or on its class, no hooks on it or on all modules.  Only then may the MLP
+    hooks on it or on all modules, no method set on it or on its class.  Only then may the MLP
     launch its kernels without those calls, or hand its forward a second argument."""
     if type(mod) is not FP8Linear:
         return False
-    d, cls = mod.__dict__, FP8Linear.__dict__
-    if (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-            or d["_backward_pre_hooks"] or "fuse_silu" in d or nn.Module.__call__ is not _MODULE_CALL):
-        return False
-    for hooks in _ALL_HOOKS:
-        if hooks:
-            return False
-    for name, method in _FP8_METHODS:
-        if name in d or cls[name] is not method:
-            return False
-    return True
+    d = mod.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                or d["_backward_pre_hooks"] or _ALL_FORWARD or _ALL_FORWARD_PRE
+                or _ALL_BACKWARD or _ALL_BACKWARD_PRE
+                or "forward" in d or "forward_prequant" in d or "quantize_input" in d
+                or "gemm_out" in d or "fuse_silu" in d
+                or FP8Linear.forward is not _FORWARD
+                or FP8Linear.forward_prequant is not _PREQUANT
+                or FP8Linear.quantize_input is not _QUANTIZE
+                or FP8Linear.gemm_out is not _GEMM or nn.Module.__call__ is not _MODULE_CALL)
 
 
 class MLP(nn.Module):
